@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/pmgpu.h"
+#include "poisson_any_ops.h"
 #include "poisson_kernels.h"
 
 namespace pmgpu {
@@ -195,6 +196,7 @@ template <typename R> struct PoissonGPU : PoissonBase {
   int Nh, Hx, Hy, Hz;
   bool allper = false;
   FftPlan pNh, pLy, pLz;
+  any::AnyPlan aNh{}, aLy{}, aLz{};   // run-time-length plans of the same lengths
   int twLx_off = 0;
   TwTable<R> tw;
   V *d_tw = nullptr;
@@ -260,6 +262,9 @@ template <typename R> struct PoissonGPU : PoissonBase {
     pLy.tw_off = tw.add(L[1]);
     pLz.tw_off = tw.add(L[2]);
     twLx_off = tw.add(L[0]);
+    make_any_plan(Nh, pNh.tw_off, aNh);
+    make_any_plan(L[1], pLy.tw_off, aLy);
+    make_any_plan(L[2], pLz.tw_off, aLz);
     PM_HIP(hipMalloc(&d_tw, tw.host.size() * sizeof(V)));
     PM_HIP(hipMemcpy(d_tw, tw.host.data(), tw.host.size() * sizeof(V), hipMemcpyHostToDevice));
     // interleaved spectral rows padded to 128 bytes so tiles align with cache lines
@@ -291,13 +296,29 @@ template <typename R> struct PoissonGPU : PoissonBase {
 
   size_t lds_bytes(int len, int lines) const { return (size_t)lines * lds_stride(len) * sizeof(V); }
 
-  // ---- generic launches -------------------------------------------------
+  // ---- launches ---------------------------------------------------------
+  // A length with a compile-time specialisation (fx_*) uses it; any other
+  // length the run-time-length passes (any_*, poisson_any.h; 160 x 100 x 125
+  // FP64 with every output 5.13 -> 1.12 ms, 44 x 56 x 45 257 -> 56 us against
+  // the kernels of poisson_kernels.h); a line that does not fit their blocks
+  // (above 4096, or three x lines of about 2400 and more) those kernels.
+  // the run-time-length plan of one of the handle's three lengths, on the
+  // twiddle table of pl (the set-up transforms have FP64 tables of their own)
+  any::AnyPlan any_plan(const FftPlan &pl) const {
+    any::AnyPlan q = pl.L == aLy.L ? aLy : (pl.L == aLz.L ? aLz : aNh);
+    if (q.L != pl.L) q.L = 0;   // no plan: not launched
+    q.tw_off = pl.tw_off;
+    return q;
+  }
   template <typename RR>
   int launch_xfwd(const void *in, void *out, int64_t cs, int64_t xs, int64_t ys, int64_t zs, int64_t o_cs,
                   int64_t o_ks, int64_t o_ys, int64_t o_zs, int ncomp, int Min, int My, int Mz, int T,
                   const FftPlan &pl, int twL, const cplx_t<RR> *twp) {
     XFwdArgs a{in, out, cs, xs, ys, zs, o_cs, o_ks, o_ys, o_zs, ncomp, Min, My, Mz, pl.L + 1, T, pl, twL};
     int f = fx_xfwd<RR>(pl.L, ncomp, a, twp, stream);
+    PM_CHECK(f >= 0, "pmgpu: x-pass launch failed");
+    if (f == 1) return 0;
+    f = any_xfwd<RR>(a, any_plan(pl), twp, stream);
     PM_CHECK(f >= 0, "pmgpu: x-pass launch failed");
     if (f == 1) return 0;
     dim3 grid((My + T - 1) / T, Mz);
@@ -312,6 +333,9 @@ template <typename R> struct PoissonGPU : PoissonBase {
                      const cplx_t<RR> *twp) {
     StridedArgs a{in, out, rs_in, rs_out, bs_in, bs_out, ncols, nin, nout, T, scale, pl, skernel};
     int f = fx_strided<RR>(pl.L, S, a, nb_y, nb_z, twp, stream);
+    PM_CHECK(f >= 0, "pmgpu: strided-pass launch failed");
+    if (f == 1) return 0;
+    f = any_strided<RR>(S, a, any_plan(pl), nb_y, nb_z, twp, stream);
     PM_CHECK(f >= 0, "pmgpu: strided-pass launch failed");
     if (f == 1) return 0;
     dim3 grid((ncols + T - 1) / T, nb_y, nb_z);
@@ -593,6 +617,7 @@ template <typename R> struct PoissonGPU : PoissonBase {
     ZArgs za = z3_args(want_psi, want_vort, reproj);
     if (record(1)) return -1;
     int fz = fx_z<R>(L[2], za, L[1], d_tw, stream);
+    if (fz == 0) fz = any_z<R>(za, aLz, L[1], d_tw, stream);
     PM_CHECK(fz >= 0, "pmgpu: z-pass launch failed");
     if (fz == 0) {
       dim3 zg((Hx + Tz - 1) / Tz, L[1]);
@@ -612,6 +637,7 @@ template <typename R> struct PoissonGPU : PoissonBase {
       XInvArgs xa{A,  reinterpret_cast<R *>(outs[f]) + off, cs, xs, ys, zs, 1, 3, H3, H3 * M[1], 3, M[0], M[1], M[2],
                   Hx, Tx, 1.0 / (double)L[0], pNh, twLx_off};
       int fxi = fx_xinv<R>(Nh, xa, d_tw, stream);
+      if (fxi == 0) fxi = any_xinv<R>(xa, aNh, d_tw, stream);
       PM_CHECK(fxi >= 0, "pmgpu: x inverse launch failed");
       if (fxi == 0) {
         dim3 grid((M[1] + Tx - 1) / Tx, M[2]);
