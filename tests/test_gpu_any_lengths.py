@@ -21,7 +21,9 @@ FREE += [((m, 6, 5), (5, m, 6), (6, 7, m))[(i + 1) % 3] for i, m in enumerate(LO
 
 
 def _solve(n, bc, ng, prec, order, kernel, reproj, psi):
-    h = 2.0 / max(n)
+    # a power of two: the kernel grid's origin is then exactly r = 0 (kernel 2
+    # divides by r^3, and a rounded origin is noise in the oracle as well)
+    h = 1.0 / 16
     xmin = [-0.5 * h * v for v in n]
     g = O.make_geom(n, ng, xmin, h, bc)
     w = blob_field(g, seed=sum(n))
