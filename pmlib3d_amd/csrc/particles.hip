@@ -1,4 +1,5 @@
 // Host side of the particle kernels: workspace, scans, C ABI.
+#include <algorithm>
 #include <cstring>
 #include <memory>
 #include <vector>
@@ -278,26 +279,70 @@ void particles_release() {
 }
 
 // ---------------------------------------------------------------- P2M
-// prec: PMGPU_FP64 (double mesh, reference arithmetic) or PMGPU_FP32 (float
-// mesh, FP32 weights, per-row partial sums Kahan-added across the stencil
-// rows); particles are FP64.
-// Order each bin's particles by id (one thread per bin), stage their records
-// (one thread per sorted particle), then gather them line by line of 64 nodes
-// along x (one wavefront per line).
+// prec: PMGPU_FP64 (double mesh) or PMGPU_FP32 (float mesh; the sums of a
+// large mesh are FP64 and rounded once, those of a small one FP32 with the row
+// partials Kahan-added); particles are FP64.
+// Order each bin's particles by id (one thread per bin), then gather them:
+// marching wavefronts (k_p2m_march), or on a small mesh one wavefront per line
+// of 64 nodes along x over staged records (k_p2m_stage, k_p2m_rows).
+//
+// A marching wavefront does the work of many line wavefronts, so a mesh needs
+// enough node lines to fill the chip with them.  Whole depositions of n^3
+// particles, lines against marches, us: M'4 FP64 64^3 95 / 101, 72^3 157 / 108,
+// 128^3 531 / 222; M'4 FP32 64^3 67 / 100, 80^3 119 / 130, 88^3 140 / 141,
+// 96^3 161 / 148, 256^3 1926 / 910; M6* FP64 64^3 245 / 283, 72^3 455 / 277,
+// 112^3 1209 / 423; M6* FP32 64^3 163 / 282, 72^3 292 / 273, 160^3 2142 / 604.
+// (Above 64 nodes along x a node line is two wavefronts, which is where the
+// lines lose but for FP32 M'4, whose records are the smallest.)
+static bool p2m_marches(const PGeom &g, int prec) {
+  const int64_t lines = (int64_t)((g.E[0] + 63) / 64) * g.E[1] * g.E[2];
+  return lines >= (prec == PMGPU_FP32 && g.ns == 4 ? 15000 : 8192);
+}
+
+// z nodes per marching wavefront.  More share a row's staging but take
+// registers: 167 for 3 (M'4), three wavefronts per SIMD; 231 for M6*, two.
+// 128^3 FP64 with 2, 3, 4: 216, 218, 220 us at each one's best chunk; M6*
+// 112 x 96 x 80 373 us with 2, 346 with 3.
+constexpr int kMarchQz = 3;
+constexpr int kMarchMostY = 32;   // longest march: its NS - 1 extra rows cost 10%; 384^3 with 32 and 96: 2.98, 2.93 ms
+
+// bytes of the staged records of np particles (0: the mesh's gather has none)
+static size_t p2m_record_bytes(const PGeom &g, int prec, int64_t np) {
+  if (np > 0 && p2m_marches(g, prec)) return 0;
+  return (prec == PMGPU_FP64 ? sizeof(double) : sizeof(float)) * PRec<double, 6>::kSlots * ((size_t)np + 1);
+}
+
 template <typename T, int NS>
-static void p2m_stage_gather(const PGeom &g, const double *xpart, const double *part, int64_t np, int *ids,
-                             PartWS &w, int nbins, T *mesh, int accumulate, hipStream_t st) {
+static void p2m_gather(const PGeom &g, const double *xpart, const double *part, int64_t np, int *ids, PartWS &w,
+                       int nbins, T *mesh, int accumulate, hipStream_t st) {
+  const int *start = w.start.as<int>();
+  const int nx = (g.E[0] + 63) / 64;
+  if (np > 0) hipLaunchKernelGGL(k_p2m_binsort, grid_for(nbins), dim3(256), 0, st, start, nbins, ids);
+  if (np > 0 && p2m_marches(g, sizeof(T) == 8 ? PMGPU_FP64 : PMGPU_FP32)) {
+    // equal segments of at most 64 nodes: with fewer than 62 a row's particles
+    // (one per bin after a remesh) take one pass of the lanes, not two
+    const int width = (g.E[0] + nx - 1) / nx, nz = (g.E[2] + kMarchQz - 1) / kMarchQz;
+    // the shortest y chunks that the chip still holds at once (a second, nearly
+    // empty round of wavefronts costs most: 160^3 FP32 chunks of 8 nodes 313 us,
+    // of 9 266 us, of 12 290 us)
+    const int64_t lines = (int64_t)nx * nz, resident = 1024 * (NS == 4 ? 3 : 2);
+    const int64_t most = resident / lines > 1 ? resident / lines : 1;
+    const int yc = (int)std::min<int64_t>((g.E[1] + most - 1) / most, kMarchMostY);
+    const int ny = (g.E[1] + yc - 1) / yc;
+    const int64_t tiles = lines * ny;
+    hipLaunchKernelGGL((k_p2m_march<T, NS, kMarchQz>), dim3((unsigned)((tiles + kMarchWaves - 1) / kMarchWaves)),
+                       dim3(64 * kMarchWaves), 0, st, g, start, ids, xpart, part, width, nx, yc, ny, tiles, mesh,
+                       accumulate);
+    return;
+  }
   // the records are planar with np + 1 records per field (the allocation
   // holds kSlots fields of np + 1)
   const int64_t rs = np + 1;
-  if (np > 0) {
-    hipLaunchKernelGGL(k_p2m_binsort, grid_for(nbins), dim3(256), 0, st, w.start.as<int>(), nbins, ids);
-    hipLaunchKernelGGL((k_p2m_stage<T, NS>), grid_for(np), dim3(256), 0, st, g, xpart, part, ids,
-                       w.start.as<int>(), nbins, w.rec.as<T>(), rs);
-  }
-  const dim3 grid((g.E[0] + 63) / 64, g.E[1], g.E[2]);
-  hipLaunchKernelGGL((k_p2m_rows<T, NS>), grid, dim3(64), 0, st, g, w.start.as<int>(), w.rec.as<T>(), rs, mesh,
-                     accumulate);
+  if (np > 0)
+    hipLaunchKernelGGL((k_p2m_stage<T, NS>), grid_for(np), dim3(256), 0, st, g, xpart, part, ids, start, nbins,
+                       w.rec.as<T>(), rs);
+  hipLaunchKernelGGL((k_p2m_rows<T, NS>), dim3(nx, g.E[1], g.E[2]), dim3(64), 0, st, g, start, w.rec.as<T>(), rs,
+                     mesh, accumulate);
 }
 
 int p2m_device(const pmgpu_geom *geom, int prec, const double *xpart, const double *part, int64_t np, void *mesh,
@@ -332,14 +377,13 @@ int p2m_device(const pmgpu_geom *geom, int prec, const double *xpart, const doub
     PM_HIP(hipGetLastError());
   }
   const int accumulate = clear ? 0 : 1;
-  const size_t rec_bytes = (prec == PMGPU_FP64 ? sizeof(double) : sizeof(float)) * PRec<double, 6>::kSlots;
-  if (w.rec.ensure(rec_bytes * ((size_t)np + 1))) return -1;
+  if (w.rec.ensure(p2m_record_bytes(g, prec, np))) return -1;
   if (prec == PMGPU_FP64) {
-    if (g.ns == 4) p2m_stage_gather<double, 4>(g, xpart, part, np, id_out, w, nbins, (double *)mesh, accumulate, st);
-    else p2m_stage_gather<double, 6>(g, xpart, part, np, id_out, w, nbins, (double *)mesh, accumulate, st);
+    if (g.ns == 4) p2m_gather<double, 4>(g, xpart, part, np, id_out, w, nbins, (double *)mesh, accumulate, st);
+    else p2m_gather<double, 6>(g, xpart, part, np, id_out, w, nbins, (double *)mesh, accumulate, st);
   } else {
-    if (g.ns == 4) p2m_stage_gather<float, 4>(g, xpart, part, np, id_out, w, nbins, (float *)mesh, accumulate, st);
-    else p2m_stage_gather<float, 6>(g, xpart, part, np, id_out, w, nbins, (float *)mesh, accumulate, st);
+    if (g.ns == 4) p2m_gather<float, 4>(g, xpart, part, np, id_out, w, nbins, (float *)mesh, accumulate, st);
+    else p2m_gather<float, 6>(g, xpart, part, np, id_out, w, nbins, (float *)mesh, accumulate, st);
   }
   PM_HIP(hipGetLastError());
   for (int d = 0; d < 3; ++d)
@@ -1040,10 +1084,9 @@ struct VStep {
     const int64_t nn = mesh_cells(g);
     PM_CHECK(cap < ((int64_t)1 << 31) && nbins < (1 << 30) && nn < ((int64_t)1 << 31),
              "pmgpu_vstep: capacity or mesh too large");
-    const size_t rec_bytes = (prec == PMGPU_FP64 ? sizeof(double) : sizeof(float)) * PRec<double, 6>::kSlots;
     if (w.key.ensure(sizeof(int) * ((size_t)cap + 1)) || w.ids.ensure(sizeof(int) * 2 * ((size_t)cap + 1)) ||
         w.count.ensure(sizeof(int) * (nbins + 1)) || w.start.ensure(sizeof(int) * (nbins + 1)) ||
-        w.rec.ensure(rec_bytes * ((size_t)cap + 1)) || w.flag.ensure(sizeof(int) * (nn + 1)) ||
+        w.rec.ensure(p2m_record_bytes(g, prec, cap)) || w.flag.ensure(sizeof(int) * (nn + 1)) ||
         w.offs.ensure(sizeof(int) * (nn + 1)))
       return -1;
     const int64_t ts = iscan_tiles(nbins > nn ? nbins : nn);
@@ -1072,11 +1115,11 @@ struct VStep {
     hipLaunchKernelGGL(k_p2m_scatter, grid_for(cap), dim3(256), 0, st, n, nbins, key, rank, w.start.as<int>(),
                        id_out);
     if (prec == PMGPU_FP64) {
-      if (g.ns == 4) p2m_stage_gather<double, 4>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
-      else p2m_stage_gather<double, 6>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
+      if (g.ns == 4) p2m_gather<double, 4>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
+      else p2m_gather<double, 6>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
     } else {
-      if (g.ns == 4) p2m_stage_gather<float, 4>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (float *)mvort(), 0, st);
-      else p2m_stage_gather<float, 6>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (float *)mvort(), 0, st);
+      if (g.ns == 4) p2m_gather<float, 4>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (float *)mvort(), 0, st);
+      else p2m_gather<float, 6>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (float *)mvort(), 0, st);
     }
     for (int d = 0; d < 3; ++d)
       if (g.bc[d] != 0) {
