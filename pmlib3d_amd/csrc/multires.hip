@@ -8,9 +8,8 @@
 // deposit in the reference: every source cell, ghosts included, spreads
 // reldx W_x W_y W_z of its value over the target stencil; parent -> patch
 // gathers W_x W_y W_z-weighted source values per target cell.  Both are
-// tensor products of per-axis operators, so the default form runs each as
-// three 1D gather passes over per-axis tap tables (HBM-streaming, no
-// atomics).  The bit-identical forms (PMGPU_M2M_EXACT=1) keep the
+// tensor products of per-axis operators, so the default form sums one axis
+// after the other, tile by tile in one kernel (no atomics).  The bit-identical forms (PMGPU_M2M_EXACT=1) keep the
 // reference's term order: the deposit as a gather in which each target cell
 // sums the terms of the source cells whose stencils cover it in the
 // reference's source-cell order (k, j, i ascending), a block of 64 target
@@ -238,138 +237,433 @@ __global__ void k_m2m_interp(const T *__restrict__ from, T *__restrict__ to, MGe
 // ---------------------------------------------------------------------------
 // Separable form (the default).  Both directions are tensor products of
 // per-axis operators: the deposit weight of a source cell onto a target cell
-// is (reldx W_x)(reldx W_y)(reldx W_z), a cell dropped on a periodic axis or
-// clamped on a free one has a zero factor on that axis, and the
-// interpolation weight is W_x W_y W_z with the same zero factors.  So each
-// direction runs as three 1D passes, each a gather along one axis over a
-// per-axis tap table, reducing (deposit) or expanding (interpolation) that
-// axis: deposit x, y, z (intermediates 1/2 and 1/4 of the patch mesh),
-// interpolation z, y, x (1/4 and 1/2).  Each pass streams its input once.
+// is (reldx W_x)(reldx W_y)(reldx W_z), a cell outside a periodic axis is
+// dropped on that axis, and the interpolation weight is W_x W_y W_z over the
+// stencil cells inside the source mesh.  So the sums run one axis after the
+// other: for an interpolation in one kernel, tile by tile with the
+// intermediate sums in LDS (the mesh's type); for a deposit, whose tiles would
+// have wide halos, in a kernel that streams the patch along z and one for x
+// and y.  A workgroup tabulates its tile's weights in LDS.
+// One direction with a kernel per axis and a table kernel per axis, and now,
+// us: 256^3 FP32 ratio 2 M'4 deposit 225, 137, interpolation 225, 97; FP64
+// 400, 247 and 404, 172; 192^3 FP32 ratio 4 M6* 177, 79 and 108, 59; 64^3 FP32
+// ratio 2 36, 19 and 25, 8.
 // The sums are regrouped against the reference's sequential loop (which
 // adds ((W_x W_y) W_z) m term by term), so the result agrees to rounding
 // (~1e-16 relative) rather than bit for bit; PMGPU_M2M_EXACT=1 selects the
 // bit-identical gathers above.
 
-constexpr int kMaxTaps = 64;  // taps of one output index on one axis (deposit: NS * ratio + 2)
+constexpr int kMThreads = 512;
+constexpr int kDownSeg = 320;   // words of a source row staged (deposit)
+// source rows staged at a time (16 and 32 FP32 rows measure the same; fewer leave LDS for more workgroups)
+template <typename T> constexpr int down_rows() { return sizeof(T) == 4 ? 16 : 8; }
+constexpr int kUpCells = 4;     // target cells per thread and plane (interpolation)
+constexpr int kMLds = 64 * 1024;
 
-struct AxisTab {
-  int *first;   // first input index (0-based, ghosts included) of each output index
-  int *count;   // number of consecutive input indices
-  double *w;    // weights, tap t of output o at w[t * stride + o] (coalesced over o)
-  int stride;
+struct M2MArgs {
+  MGeom f, t;
+  double reldx;
+  int clear;
+  int W, H, D;        // target cells of a tile along x, y and of a march along z
+  int nx, ny, nz;     // tiles
+  int cap[3];         // staged source indices per axis (deposit: candidates; interpolation: source cells)
+  int taps[2];        // most taps of a target index along x, y (deposit)
+  int rows;           // source rows per pass (deposit)
+  int stage_bytes;    // LDS of the rows and, before, of the staged indices
 };
 
-// Tap table of axis d.  Deposit (src finer): output index T (reference
-// numbering) takes the source indices whose base b satisfies b - off <= T <=
-// b - off + NS - 1, weight reldx W_{T - b + off}, zero for a cell outside
-// the box on a periodic axis.  Interpolation (src coarser): output index T
-// takes the stencil slots inside the source mesh, weight W_s.
-template <int NS>
-__global__ void k_m2m_table(MGeom src, MGeom dst, int d, int deposit, double reldx, AxisTab tab) {
-  constexpr int off = NS == 6 ? 2 : 1;
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= dst.E[d]) return;
-  const int T = o + 1 - dst.ng[d];
-  double *w = tab.w + o;
-  const int ws = tab.stride;
-  int first = 0, n = 0;
-  if (deposit) {
-    int ilo, ihi;
-    src_range(src, dst, d, T + off - NS + 1, T + off, ilo, ihi);
-    for (int i = ilo; i <= ihi; ++i) {
-      const double p = __dadd_rn(src.xmin[d], __dmul_rn(__dadd_rn((double)(i - 1), 0.5), src.dx[d]));
-      const int b = cell_index(p, dst.xmin[d], dst.c1dx[d]);
-      const int s = T - b + off;
-      if (s < 0 || s >= NS) continue;
-      if (n == 0) first = i - 1 + src.ng[d];
-      if (n >= kMaxTaps) break;
-      const bool live = !(dst.bc[d] != 0 && (p < dst.xmin[d] || p > dst.xmax[d]));
-      const double dd = stencil_offset(p, dst.xmin[d], dst.dx[d], b, dst.c1dx[d]);
-      w[ws * n++] = live ? __dmul_rn(reldx, weight(NS == 6, s, dd)) : 0.0;
-    }
-  } else {
-    const double p = __dadd_rn(dst.xmin[d], __dmul_rn(__dadd_rn((double)(T - 1), 0.5), dst.dx[d]));
-    const int b = cell_index(p, src.xmin[d], src.c1dx[d]);
-    const double dd = stencil_offset(p, src.xmin[d], src.dx[d], b, src.c1dx[d]);
-    for (int s = 0; s < NS; ++s) {
-      const int q = b - off + s;
-      if (q < 1 - src.ng[d] || q > src.ncell[d] + src.ng[d]) continue;
-      if (n == 0) first = q - 1 + src.ng[d];
-      w[ws * n++] = weight(NS == 6, s, dd);
-    }
-  }
-  tab.first[o] = first;
-  tab.count[o] = n;
+// a tile's position: workgroups of one XCD take neighbouring tiles (x fastest,
+// then y, then z), whose source cells they share in that XCD's L2
+__device__ __forceinline__ void m2m_tile(const M2MArgs &a, int *o, int *n) {
+  const int64_t lt = xcd_tile(blockIdx.x, gridDim.x);
+  o[0] = (int)(lt % a.nx) * a.W;
+  o[1] = (int)((lt / a.nx) % a.ny) * a.H;
+  o[2] = (int)(lt / ((int64_t)a.nx * a.ny)) * a.D;
+  n[0] = min(a.W, a.t.E[0] - o[0]);
+  n[1] = min(a.H, a.t.E[1] - o[1]);
+  n[2] = min(a.D, a.t.E[2] - o[2]);
 }
 
-struct PassArgs {
-  int d;             // axis of the pass
-  int Ein[3], Eout[3];
-  AxisTab tab;
-  int final_pass;    // writes the caller's mesh: clear / accumulate / skip rules apply
-  int clear;
-  int skip_bc[3];    // final interpolation pass: periodic axes whose ghost cells are not written
-  int nc[3], ng[3];  // (of the output mesh, for the skip rule)
+// i / n of the items of a tile, with inv = 1 / n (exact: i < 2^16, n < 2^10,
+// and (i + 1/2) / n is 1 / 2n away from a whole number)
+__device__ __forceinline__ int quot(int i, float inv) { return (int)(((float)i + 0.5f) * inv); }
+
+// the three components of a cell
+template <typename T> struct Cell3 {
+  T x, y, z;
 };
 
-// One 1D pass: grid (ceil(Eout_x Eout_y / 256), Eout_z), a thread per
-// output cell (all three components).
-template <typename Tin, typename Tout>
-__global__ void __launch_bounds__(256) k_m2m_pass(const Tin *__restrict__ in, Tout *__restrict__ out, PassArgs a) {
-  // XCD-aware order: the workgroups of one XCD take consecutive (xy, z)
-  // tiles, so a z pass's taps on neighbouring planes are shared in its L2
-  const int64_t lt = xcd_tile(blockIdx.x + (int64_t)gridDim.x * blockIdx.y, (int64_t)gridDim.x * gridDim.y);
-  const int bx = (int)(lt % gridDim.x), bz = (int)(lt / gridDim.x);
-  const int xy = (int)(bx * blockDim.x + threadIdx.x);
-  if (xy >= a.Eout[0] * a.Eout[1]) return;
-  int x[3] = {xy % a.Eout[0], xy / a.Eout[0], bz};
-  const int64_t c = (int64_t)x[0] + (int64_t)a.Eout[0] * (x[1] + (int64_t)a.Eout[1] * x[2]);
-  const int64_t sin[3] = {3, 3 * (int64_t)a.Ein[0], 3 * (int64_t)a.Ein[0] * a.Ein[1]};
-  {
-    if (a.final_pass) {
-      bool skip = false;
+// words of a mesh line at a time (a line starts at any word)
+template <typename T, int V> struct alignas(sizeof(T)) Words {
+  T v[V];
+};
+
+// Patch -> parent, the sums along z: a thread owns V words of the mesh's planes
+// and marches up the source planes that reach its D target planes, adding each
+// to the NS target planes it reaches (a window in registers, stored as the
+// planes leave it), four planes' loads in flight.  Reads the patch once but for
+// the NS - 1 planes on either side of a march, and writes 1 / ratio of it:
+// bound by memory, 256^3 FP32 70 us for 317 MB.
+template <typename T, int NS, int V>
+__global__ void __launch_bounds__(256) k_m2m_down_z(const T *__restrict__ from, T *__restrict__ mid, M2MArgs a) {
+  constexpr int off = NS == 6 ? 2 : 1;
+  extern __shared__ double m2m_lds[];
+  const MGeom &f = a.f, &t = a.t;
+  const int64_t words = 3 * (int64_t)f.E[0] * f.E[1];
+  const int o = (int)blockIdx.y * a.D, n = min(a.D, t.E[2] - o);
+  double *const zw = m2m_lds;
+  int *const zb = reinterpret_cast<int *>(zw + (size_t)a.cap[2] * NS), *const zl = zb + a.cap[2];
+  const int T0 = o + 1 - t.ng[2], T1 = T0 + n - 1;
+  int zlo, zhi;
+  src_range(f, t, 2, T0 + off - NS + 1, T1 + off, zlo, zhi);
+  const int nzs = max(min(zhi - zlo + 1, a.cap[2]), 0);
+  for (int q = threadIdx.x; q < nzs; q += blockDim.x) {
+    unsigned char live;
+    stage_src<NS>(f, t, 2, zlo + q, a.reldx, zb[q], live, zw + (size_t)q * NS);
+    zl[q] = live;
+  }
+  __syncthreads();
+  // (the last thread's words may be its neighbour's too: the same values)
+  const int64_t w0 = min(V * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), words - V);
+  if (V * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >= words) return;
+  const int q0 = lower_bound_b(zb, nzs, T0 + off - NS + 1), q1 = lower_bound_b(zb, nzs, T1 + off + 1);
+  const T *src = from + w0 + words * (zlo - 1 + f.ng[2]);
+  double acc[NS][V];
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
-        if (a.skip_bc[q] && (x[q] < a.ng[q] || x[q] >= a.ng[q] + a.nc[q])) skip = true;
-      if (skip) {
-        if (a.clear) out[3 * c] = out[3 * c + 1] = out[3 * c + 2] = (Tout)0;
-        return;
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int c = 0; c < V; ++c) acc[s][c] = 0.0;
+  int cur = T0 - NS + 1;   // target plane of acc[0]
+  auto advance = [&] {
+    if (cur >= T0) {
+      Words<T, V> r;
+#pragma unroll
+      for (int c = 0; c < V; ++c) r.v[c] = (T)acc[0][c];
+      *reinterpret_cast<Words<T, V> *>(mid + w0 + words * (cur - 1 + t.ng[2])) = r;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int c = 0; c < V; ++c) acc[s][c] = s + 1 < NS ? acc[s + 1][c] : 0.0;
+    ++cur;
+  };
+  for (int q = q0; q < q1; q += 4) {
+    Words<T, V> v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = *reinterpret_cast<const Words<T, V> *>(src + words * min(q + u, q1 - 1));
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (q + u < q1 && zl[q + u]) {
+        const int b = __builtin_amdgcn_readfirstlane(zb[q + u]);
+        while (cur < b - off) advance();
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const double w = zw[(size_t)(q + u) * NS + s];
+#pragma unroll
+          for (int c = 0; c < V; ++c) acc[s][c] = __fma_rn(w, (double)v[u].v[c], acc[s][c]);
+        }
+      }
+  }
+  while (cur <= T1) advance();
+}
+
+// Patch -> parent, the sums along x and y of the planes summed along z.  A
+// workgroup owns W x H target columns; a plane's source rows under them are
+// copied into LDS (a wavefront per row, the next rows' loads in flight while
+// these are summed), summed along x into LDS again, and along y in registers.
+// What bounds it: LDS, NS ratio words per sum on both axes: 256^3 FP32 79 us.
+// (Rows summed along x straight from memory, their loads waited for tap by tap,
+// and all three axes in one march: 164 us against 149 for both kernels at 256^3
+// FP32, 621 against 77 at 192^3 ratio 4 M6*.)
+template <typename T, int NS>
+__global__ void __launch_bounds__(kMThreads) k_m2m_down_xy(const T *__restrict__ mid, T *__restrict__ to, M2MArgs a) {
+  constexpr int off = NS == 6 ? 2 : 1, kWaves = kMThreads / 64, RK = down_rows<T>() / kWaves, SK = kDownSeg / 64;
+  extern __shared__ double m2m_lds[];
+  const MGeom &f = a.f, &t = a.t;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int o[3], n[3];
+  m2m_tile(a, o, n);
+  // LDS: source rows and x sums (first the staged indices of one axis: weights,
+  // bases, live flags), tap weights of x and y; first taps and counts
+  double *const st_w = m2m_lds;
+  T *const raw = reinterpret_cast<T *>(m2m_lds), *const X = raw + down_rows<T>() * kDownSeg;
+  double *const wx = m2m_lds + a.stage_bytes / 8, *const wy = wx + a.taps[0] * a.W;
+  int *const fx = reinterpret_cast<int *>(wy + a.taps[1] * a.H), *const cx = fx + a.W;
+  int *const fy = cx + a.W, *const cy = fy + a.H;
+
+  int lo[2], len[2];   // source cells under the tile
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const int T0 = o[d] + 1 - t.ng[d], nt = n[d], cap = a.cap[d], w0 = d == 0 ? a.W : a.H;
+    int *const sb = reinterpret_cast<int *>(st_w + (size_t)cap * NS), *const sl = sb + cap;
+    int *const first = d == 0 ? fx : fy, *const count = d == 0 ? cx : cy;
+    double *const wt = d == 0 ? wx : wy;
+    int ilo, ihi;
+    src_range(f, t, d, T0 + off - NS + 1, T0 + nt - 1 + off, ilo, ihi);
+    const int ns = max(min(ihi - ilo + 1, cap), 0), i0 = ilo - 1 + f.ng[d];
+    for (int q = tid; q < ns; q += kMThreads) {
+      unsigned char live;
+      stage_src<NS>(f, t, d, ilo + q, a.reldx, sb[q], live, st_w + (size_t)q * NS);
+      sl[q] = live;
+    }
+    __syncthreads();
+    const int b0 = lower_bound_b(sb, ns, T0 + off - NS + 1), b1 = lower_bound_b(sb, ns, T0 + nt + off);
+    lo[d] = __builtin_amdgcn_readfirstlane(i0 + b0);
+    len[d] = __builtin_amdgcn_readfirstlane(d == 0 ? min(b1 - b0, kDownSeg / 3) : b1 - b0);
+    for (int q = tid; q < nt; q += kMThreads) {
+      int q0 = lower_bound_b(sb, ns, T0 + q + off - NS + 1), q1 = lower_bound_b(sb, ns, T0 + q + off + 1);
+      while (q0 < q1 && !sl[q0]) ++q0;
+      while (q0 < q1 && !sl[q1 - 1]) --q1;
+      first[q] = q0 - b0;
+      count[q] = max(min(min(q1 - q0, a.taps[d]), len[d] - (q0 - b0)), 0);
+    }
+    __syncthreads();
+    for (int i = tid; i < a.taps[d] * nt; i += kMThreads) {
+      const int k = i / nt, q = i - k * nt;
+      if (k < count[q]) {
+        const int e = first[q] + b0 + k;
+        wt[k * w0 + q] = st_w[(size_t)e * NS + (T0 + q - sb[e] + off)];
       }
     }
-    const int o = x[a.d];
-    const int first = a.tab.first[o], cnt = a.tab.count[o];
-    const double *w = a.tab.w + o;
-    const int ws = a.tab.stride;
-    x[a.d] = first;
-    const Tin *p = in + sin[0] * x[0] + sin[1] * x[1] + sin[2] * x[2];
-    const int64_t st = sin[a.d];
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int t = 0; t < cnt; ++t) {
-      const double wt = w[t * ws];
-      s0 += wt * (double)p[0];
-      s1 += wt * (double)p[1];
-      s2 += wt * (double)p[2];
-      p += st;
+    __syncthreads();
+  }
+  const int ty = tid / n[0], tx = tid - ty * n[0];
+  const bool mine = ty < n[1];
+  const int my0 = mine ? fy[ty] : 0, my1 = my0 + (mine ? cy[ty] : 0);
+  const int seg = 3 * len[0], rows = len[1], chunk = min(a.rows, down_rows<T>());
+  const int plane = a.rows * a.W;   // LDS words of an x sum's component
+  const int64_t sy = 3 * (int64_t)f.E[0], sz = sy * f.E[1];
+  const T *src = mid + sy * lo[1] + 3 * (int64_t)lo[0] + sz * o[2];
+  auto put = [&](int q, double v0, double v1, double v2) {
+    if (!mine) return;
+    Cell3<T> *p = reinterpret_cast<Cell3<T> *>(to) + (int64_t)(o[0] + tx) +
+                  (int64_t)t.E[0] * ((o[1] + ty) + (int64_t)t.E[1] * (o[2] + q));
+    if (!a.clear) {
+      const Cell3<T> v = *p;
+      v0 += (double)v.x;
+      v1 += (double)v.y;
+      v2 += (double)v.z;
     }
-    if (a.final_pass && !a.clear) {
-      s0 += (double)out[3 * c];
-      s1 += (double)out[3 * c + 1];
-      s2 += (double)out[3 * c + 2];
+    *p = Cell3<T>{(T)v0, (T)v1, (T)v2};
+  };
+  if (seg <= 0 || rows <= 0) {   // no source cell reaches the tile
+    for (int q = 0; q < n[2]; ++q) put(q, 0.0, 0.0, 0.0);
+    return;
+  }
+  T reg[RK][SK];
+  auto load = [&](int q, int r0) {
+#pragma unroll
+    for (int i = 0; i < RK; ++i) {
+      const T *p = src + sz * q + sy * min(r0 + wave + kWaves * i, rows - 1);
+#pragma unroll
+      for (int k = 0; k < SK; ++k) reg[i][k] = p[min(lane + 64 * k, seg - 1)];
     }
-    out[3 * c] = (Tout)s0;
-    out[3 * c + 1] = (Tout)s1;
-    out[3 * c + 2] = (Tout)s2;
+  };
+  const float inv = 1.0f / (float)n[0];
+  load(0, 0);
+  double v0 = 0.0, v1 = 0.0, v2 = 0.0;
+  for (int q = 0, r0 = 0; q < n[2];) {
+    const int m = min(chunk, rows - r0);
+#pragma unroll
+    for (int i = 0; i < RK; ++i)
+#pragma unroll
+      for (int k = 0; k < SK; ++k) raw[(wave + kWaves * i) * kDownSeg + lane + 64 * k] = reg[i][k];
+    __syncthreads();
+    const bool last = r0 + m >= rows;
+    const int qn = last ? q + 1 : q, rn = last ? 0 : r0 + m;
+    if (qn < n[2]) load(qn, rn);
+    for (int i = tid; i < m * n[0]; i += kMThreads) {
+      const int r = quot(i, inv), x = i - r * n[0];
+      const T *p = raw + r * kDownSeg + 3 * fx[x];
+      const double *w = wx + x;
+      const int cnt = cx[x];
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+      for (int e = 0; e < cnt; ++e) {
+        const double wt = w[e * a.W];
+        s0 = __fma_rn(wt, (double)p[3 * e], s0);
+        s1 = __fma_rn(wt, (double)p[3 * e + 1], s1);
+        s2 = __fma_rn(wt, (double)p[3 * e + 2], s2);
+      }
+      T *xs = X + r * a.W + x;
+      xs[0] = (T)s0;
+      xs[plane] = (T)s1;
+      xs[2 * plane] = (T)s2;
+    }
+    __syncthreads();
+    const int e1 = min(my1, r0 + m);
+    for (int e = max(my0, r0); e < e1; ++e) {
+      const double wt = wy[(e - my0) * a.H + ty];
+      const T *xs = X + (e - r0) * a.W + tx;
+      v0 = __fma_rn(wt, (double)xs[0], v0);
+      v1 = __fma_rn(wt, (double)xs[plane], v1);
+      v2 = __fma_rn(wt, (double)xs[2 * plane], v2);
+    }
+    if (last) {
+      put(q, v0, v1, v2);
+      v0 = v1 = v2 = 0.0;
+    }
+    q = qn;
+    r0 = rn;
   }
 }
 
-// Intermediate meshes and tap tables, grown on demand, kept until
-// pmgpu_finalize (one set per process: calls that overlap race).
+// Parent -> patch.  A workgroup owns W x H target columns and D target planes:
+// for each plane the source cells under it are summed along z into LDS, those
+// along y into LDS again, and those along x stored.
+// What bounds it: the patch's store (256^3 FP32 211 MB, 41 us at the card's
+// copy rate) and the sums along x, 6 NS conversions and multiply-adds per
+// target cell and as many LDS reads: 97 us.
+template <typename T, int NS>
+__global__ void __launch_bounds__(kMThreads) k_m2m_up(const T *__restrict__ from, T *__restrict__ to, M2MArgs a) {
+  constexpr int off = NS == 6 ? 2 : 1;
+  extern __shared__ double m2m_lds[];
+  const MGeom &f = a.f, &t = a.t;
+  const int tid = threadIdx.x;
+  int o[3], n[3];
+  m2m_tile(a, o, n);
+  // LDS: weights per target index, z sums, y sums, first source cells
+  const int len[3] = {a.W, a.H, a.D};
+  double *const wx = m2m_lds, *const wy = wx + NS * len[0], *const zw = wy + NS * len[1];
+  T *const A = reinterpret_cast<T *>(zw + NS * len[2]);
+  const int ca = a.cap[0] * a.cap[1], cb = a.cap[0] * a.H;
+  T *const B = A + 3 * ca;
+  int *const bx = reinterpret_cast<int *>(m2m_lds) + a.stage_bytes / 4, *const by = bx + len[0], *const zb = by + len[1];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double *const w = d == 0 ? wx : d == 1 ? wy : zw;
+    int *const base = d == 0 ? bx : d == 1 ? by : zb;
+    for (int q = tid; q < n[d]; q += kMThreads) {
+      const double p = __dadd_rn(t.xmin[d], __dmul_rn(__dadd_rn((double)(o[d] + q - t.ng[d]), 0.5), t.dx[d]));
+      const int b = cell_index(p, f.xmin[d], f.c1dx[d]);
+      const double dd = stencil_offset(p, f.xmin[d], f.dx[d], b, f.c1dx[d]);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) w[s * len[d] + q] = weight(NS == 6, s, dd);
+      base[q] = b - off - 1 + f.ng[d];   // (0-based; the stencil may leave the source mesh)
+    }
+  }
+  __syncthreads();
+  // source cells under the tile (bases are non-decreasing)
+  const int cx0 = bx[0], cy0 = by[0];
+  const int cw = min(bx[n[0] - 1] - cx0 + NS, a.cap[0]), ch = min(by[n[1] - 1] - cy0 + NS, a.cap[1]);
+  const float inv = 1.0f / (float)cw;
+  const int64_t sy = 3 * (int64_t)f.E[0], sz = sy * f.E[1];
+  auto skips = [&](int d, int x) { return t.bc[d] != 0 && (x < t.ng[d] || x >= t.ng[d] + t.ncell[d]); };
+  // the thread's target cells
+  int off_b[kUpCells], tx[kUpCells], ty[kUpCells];
+#pragma unroll
+  for (int k = 0; k < kUpCells; ++k) {
+    const int i = tid + k * kMThreads;
+    ty[k] = i / n[0];
+    tx[k] = i - ty[k] * n[0];
+    if (ty[k] >= n[1]) ty[k] = -1;
+    off_b[k] = ty[k] < 0 ? 0 : ty[k] * a.cap[0] + bx[tx[k]] - cx0;
+  }
+  for (int q = 0; q < n[2]; ++q) {
+    const int z = o[2] + q;
+    const int z0 = __builtin_amdgcn_readfirstlane(zb[q]);
+    double w[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) w[s] = zw[s * len[2] + q];
+    for (int i = tid; i < cw * ch; i += kMThreads) {
+      const int y = quot(i, inv), x = i - y * cw;
+      const int gx = cx0 + x, gy = cy0 + y;
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+      if (gx >= 0 && gx < f.E[0] && gy >= 0 && gy < f.E[1]) {
+        Cell3<T> v[NS];
+        const T *p = from + sy * gy + 3 * (int64_t)gx;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          v[s] = *reinterpret_cast<const Cell3<T> *>(p + sz * min(max(z0 + s, 0), f.E[2] - 1));
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          if (z0 + s >= 0 && z0 + s < f.E[2]) {
+            s0 = __fma_rn(w[s], (double)v[s].x, s0);
+            s1 = __fma_rn(w[s], (double)v[s].y, s1);
+            s2 = __fma_rn(w[s], (double)v[s].z, s2);
+          }
+      }
+      T *p = A + y * a.cap[0] + x;
+      p[0] = (T)s0;
+      p[ca] = (T)s1;
+      p[2 * ca] = (T)s2;
+    }
+    __syncthreads();
+    for (int i = tid; i < cw * n[1]; i += kMThreads) {
+      const int y = quot(i, inv), x = i - y * cw;
+      const T *p = A + (by[y] - cy0) * a.cap[0] + x;
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const double wt = wy[s * len[1] + y];
+        s0 = __fma_rn(wt, (double)p[s * a.cap[0]], s0);
+        s1 = __fma_rn(wt, (double)p[s * a.cap[0] + ca], s1);
+        s2 = __fma_rn(wt, (double)p[s * a.cap[0] + 2 * ca], s2);
+      }
+      T *r = B + y * a.cap[0] + x;
+      r[0] = (T)s0;
+      r[cb] = (T)s1;
+      r[2 * cb] = (T)s2;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kUpCells; ++k)
+      if (ty[k] >= 0) {
+        const bool skip = skips(0, o[0] + tx[k]) || skips(1, o[1] + ty[k]) || skips(2, z);
+        const T *p = B + off_b[k];
+        Cell3<T> *r = reinterpret_cast<Cell3<T> *>(to) + (int64_t)(o[0] + tx[k]) +
+                      (int64_t)t.E[0] * ((o[1] + ty[k]) + (int64_t)t.E[1] * z);
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const double wt = wx[s * len[0] + tx[k]];
+          s0 = __fma_rn(wt, (double)p[s], s0);
+          s1 = __fma_rn(wt, (double)p[s + cb], s1);
+          s2 = __fma_rn(wt, (double)p[s + 2 * cb], s2);
+        }
+        if (a.clear) {
+          *r = skip ? Cell3<T>{0, 0, 0} : Cell3<T>{(T)s0, (T)s1, (T)s2};
+        } else if (!skip) {
+          const Cell3<T> v = *r;
+          *r = Cell3<T>{(T)(s0 + (double)v.x), (T)(s1 + (double)v.y), (T)(s2 + (double)v.z)};
+        }
+      }
+  }
+}
+
+// Tile of a deposit or an interpolation: W x H target columns, W at most
+// most_w, W H at most `most` and equal along each axis, the ones that sum the
+// fewest source cells (their halos count) and leave the fewest lanes without a
+// column; D target planes so that the chip has kMTiles workgroups.
+constexpr int kMTiles = 1024;
+void m2m_tiles(M2MArgs &a, int most, int most_w, int halo) {
+  double best = 0.0;
+  for (int nx = 1; nx <= a.t.E[0]; ++nx) {
+    const int W = (a.t.E[0] + nx - 1) / nx;
+    if (W > std::min(most, most_w)) continue;
+    if (W < 8 && best > 0.0) break;
+    int H = std::min(std::min(most / W, a.t.E[1]), 64);
+    const int ny = (a.t.E[1] + H - 1) / H;
+    H = (a.t.E[1] + ny - 1) / ny;
+    const double cost = (double)nx * ny * ((double)(H + halo) * (W + halo) + most);
+    if (best == 0.0 || cost < best) {
+      best = cost;
+      a.W = W;
+      a.H = H;
+    }
+  }
+  a.nx = (a.t.E[0] + a.W - 1) / a.W;
+  a.ny = (a.t.E[1] + a.H - 1) / a.H;
+  const int64_t want = std::max<int64_t>(1, kMTiles / ((int64_t)a.nx * a.ny));
+  a.D = (int)std::min<int64_t>((a.t.E[2] + want - 1) / want, 32);
+  a.nz = (a.t.E[2] + a.D - 1) / a.D;
+}
+
+// Intermediate mesh of the deposit, grown on demand, kept until
+// pmgpu_finalize (one per process: calls that overlap race).
 struct M2MWS {
-  void *a = nullptr, *b = nullptr;
-  size_t na = 0, nb = 0;
-  int *first = nullptr, *count = nullptr;
-  double *w = nullptr;
-  int ntab = 0;
+  void *a = nullptr;
+  size_t na = 0;
 };
 M2MWS g_m2m;
 std::mutex g_m2m_mu;
@@ -384,92 +678,121 @@ int grow(void *&p, size_t &have, size_t want) {
   return 0;
 }
 
+// 1: not a mesh for these kernels
+template <typename T, int NS> int m2m_down(M2MArgs &a, const T *src, T *dst, hipStream_t st) {
+  int ratio[3];
+  for (int d = 0; d < 3; ++d) ratio[d] = std::max(1, (int)std::ceil(a.t.dx[d] / a.f.dx[d] - 1e-6));
+  // z: V words per thread, D planes per march
+  constexpr int V = 16 / sizeof(T);
+  const int64_t words = 3 * (int64_t)a.f.E[0] * a.f.E[1];
+  if (words < V) return 1;
+  const size_t bytes = sizeof(T) * (size_t)words * a.t.E[2];
+  std::lock_guard<std::mutex> lock(g_m2m_mu);
+  if (grow(g_m2m.a, g_m2m.na, bytes)) return -1;
+  T *mid = static_cast<T *>(g_m2m.a);
+  const int64_t bx = (words + V * 256 - 1) / (V * 256);
+  const int64_t marches = std::max<int64_t>(1, kMTiles / bx);
+  a.D = (int)std::min<int64_t>((a.t.E[2] + marches - 1) / marches, 32);
+  a.cap[2] = (a.D + NS + 2) * ratio[2] + 8;
+  const dim3 zgrid((unsigned)bx, (a.t.E[2] + a.D - 1) / a.D);
+  hipLaunchKernelGGL((k_m2m_down_z<T, NS, V>), zgrid, dim3(256),
+                     a.cap[2] * (sizeof(double) * NS + 2 * sizeof(int)), st, src, mid, a);
+  PM_HIP(hipGetLastError());
+  // x and y: the widest tile whose source cells ((W + NS - 1) ratio and one for
+  // the ends) fit the staged rows, and its sums LDS
+  size_t lds = 0;
+  for (int mw = (kDownSeg / 3 - 2) / ratio[0] - (NS - 1); mw > 0; --mw) {
+    m2m_tiles(a, kMThreads, mw, NS - 1);
+    const int n[2] = {a.W, a.H};
+    for (int d = 0; d < 2; ++d) {
+      a.cap[d] = (n[d] + NS + 2) * ratio[d] + 8;
+      a.taps[d] = NS * ratio[d] + 2;
+    }
+    a.rows = std::min(down_rows<T>(), a.cap[1]);
+    const size_t stage = std::max(a.cap[0], a.cap[1]) * (sizeof(double) * NS + 2 * sizeof(int));
+    a.stage_bytes =
+        (int)((std::max(sizeof(T) * (down_rows<T>() * kDownSeg + 3 * (size_t)a.rows * a.W), stage) + 7) / 8 * 8);
+    lds = a.stage_bytes + sizeof(double) * ((size_t)a.taps[0] * a.W + (size_t)a.taps[1] * a.H) +
+          sizeof(int) * 2 * ((size_t)a.W + a.H);
+    if (lds <= kMLds) break;
+  }
+  if (lds == 0 || lds > kMLds) return 1;
+  const int64_t tiles = (int64_t)a.nx * a.ny * a.nz;
+  PM_CHECK(tiles < ((int64_t)1 << 31), "pmgpu_interp_mesh_mesh: mesh too large");
+  hipLaunchKernelGGL((k_m2m_down_xy<T, NS>), dim3((unsigned)tiles), dim3(kMThreads), lds, st, (const T *)mid, dst, a);
+  PM_HIP(hipGetLastError());
+  return 0;
+}
+
+template <typename T, int NS> int m2m_up(M2MArgs &a, const T *src, T *dst, hipStream_t st) {
+  // the largest tile whose sums fit in LDS; none for a mesh much finer along
+  // another axis than along x
+  size_t lds = 0;
+  for (int most = kMThreads * kUpCells; most >= 64; most /= 2) {
+    m2m_tiles(a, most, 128, 0);
+    const int n[2] = {a.W, a.H};
+    // (bases n - 1 spacings apart differ by that many source cells, rounded up)
+    double c[2];
+    for (int d = 0; d < 2; ++d) c[d] = std::ceil(n[d] * a.t.dx[d] / a.f.dx[d] * (1.0 + 1e-9)) + NS + 1;
+    const double w = sizeof(double) * NS * ((double)a.W + a.H + a.D);
+    lds = 0;
+    if (w + 3.0 * sizeof(T) * c[0] * (c[1] + a.H) > kMLds) continue;
+    for (int d = 0; d < 2; ++d) a.cap[d] = (int)c[d];
+    a.stage_bytes = (int)(w + 3 * sizeof(T) * a.cap[0] * (a.cap[1] + a.H) + 7) / 8 * 8;
+    lds = a.stage_bytes + sizeof(int) * ((size_t)a.W + a.H + a.D);
+    break;
+  }
+  if (lds == 0) return 1;
+  const int64_t tiles = (int64_t)a.nx * a.ny * a.nz;
+  PM_CHECK(tiles < ((int64_t)1 << 31), "pmgpu_interp_mesh_mesh: mesh too large");
+  hipLaunchKernelGGL((k_m2m_up<T, NS>), dim3((unsigned)tiles), dim3(kMThreads), lds, st, src, dst, a);
+  PM_HIP(hipGetLastError());
+  return 0;
+}
+
+// the ghost layers of periodic axes after a deposit (added onto their images,
+// :1380-1386, pmlib_mesh_map_ghost with incl_edges, op add) or an
+// interpolation (copied from their images, :2057-2063, op replace)
+template <typename T> int m2m_periodic(const MGeom &t, bool deposit, T *dst, hipStream_t st) {
+  PGeom pg{};
+  for (int d = 0; d < 3; ++d) {
+    pg.ncell[d] = t.ncell[d];
+    pg.ngl[d] = t.ng[d];
+    pg.E[d] = t.E[d];
+  }
+  for (int d = 0; d < 3; ++d)
+    if (t.bc[d] != 0) {
+      if (deposit)
+        hipLaunchKernelGGL(k_halo_add<T>, dim3(256), dim3(256), 0, st, dst, pg, d);
+      else
+        hipLaunchKernelGGL(k_ghost_fill<T>, dim3(1024), dim3(256), 0, st, dst, t.E[0], t.E[1], t.E[2], d, t.ncell[d],
+                           t.ng[d], 3);
+      PM_HIP(hipGetLastError());
+    }
+  return 0;
+}
+
+template <typename T>
+int m2m_exact(const MGeom &f, const MGeom &t, int ns, const void *from, void *to, int clear, hipStream_t st);
+
 template <typename T>
 int m2m_separable(const MGeom &f, const MGeom &t, int ns, const void *from, void *to, int clear, hipStream_t st) {
   const bool deposit = f.dx[0] / t.dx[0] <= 0.9999;
-  const double reldx = f.dx[0] / t.dx[0];
   for (int d = 0; d < 3; ++d)
     PM_CHECK(!deposit || t.dx[d] / f.dx[d] <= (double)kMaxRatio + 1e-9,
              "pmgpu_interp_mesh_mesh: cell size ratios above 8 are not supported");
-  // the three shapes: deposit reduces x, y, z in turn; interpolation expands z, y, x
-  int E1[3], E2[3];
-  const int order[3] = {deposit ? 0 : 2, 1, deposit ? 2 : 0};
-  for (int q = 0; q < 3; ++q) E1[q] = f.E[q];
-  E1[order[0]] = t.E[order[0]];
-  for (int q = 0; q < 3; ++q) E2[q] = E1[q];
-  E2[order[1]] = t.E[order[1]];
-  const size_t bytes1 = sizeof(T) * 3 * (size_t)E1[0] * E1[1] * E1[2];
-  const size_t bytes2 = sizeof(T) * 3 * (size_t)E2[0] * E2[1] * E2[2];
-  const int emax = std::max(t.E[0], std::max(t.E[1], t.E[2]));
-  std::lock_guard<std::mutex> lock(g_m2m_mu);
-  if (grow(g_m2m.a, g_m2m.na, bytes1) || grow(g_m2m.b, g_m2m.nb, bytes2)) return -1;
-  if (g_m2m.ntab < emax) {
-    if (g_m2m.first) (void)hipFree(g_m2m.first);
-    if (g_m2m.count) (void)hipFree(g_m2m.count);
-    if (g_m2m.w) (void)hipFree(g_m2m.w);
-    g_m2m.first = g_m2m.count = nullptr;
-    g_m2m.w = nullptr;
-    g_m2m.ntab = 0;
-    PM_HIP(hipMalloc(&g_m2m.first, sizeof(int) * 3 * emax));
-    PM_HIP(hipMalloc(&g_m2m.count, sizeof(int) * 3 * emax));
-    PM_HIP(hipMalloc(&g_m2m.w, sizeof(double) * 3 * (size_t)emax * kMaxTaps));
-    g_m2m.ntab = emax;
-  }
-  AxisTab tabs[3];
-  for (int d = 0; d < 3; ++d) {
-    tabs[d] = AxisTab{g_m2m.first + d * emax, g_m2m.count + d * emax, g_m2m.w + (size_t)d * emax * kMaxTaps,
-                      emax};
-    const int blocks = (t.E[d] + 127) / 128;
-    if (ns == 6)
-      hipLaunchKernelGGL(k_m2m_table<6>, dim3(blocks), dim3(128), 0, st, f, t, d, (int)deposit, reldx, tabs[d]);
-    else
-      hipLaunchKernelGGL(k_m2m_table<4>, dim3(blocks), dim3(128), 0, st, f, t, d, (int)deposit, reldx, tabs[d]);
-    PM_HIP(hipGetLastError());
-  }
-  const void *ins[3] = {from, g_m2m.a, g_m2m.b};
-  void *outs[3] = {g_m2m.a, g_m2m.b, to};
-  const int *Eins[3] = {f.E, E1, E2};
-  const int *Eouts[3] = {E1, E2, t.E};
-  for (int q = 0; q < 3; ++q) {
-    PassArgs a{};
-    a.d = order[q];
-    for (int k = 0; k < 3; ++k) {
-      a.Ein[k] = Eins[q][k];
-      a.Eout[k] = Eouts[q][k];
-      a.skip_bc[k] = (!deposit && t.bc[k] != 0) ? 1 : 0;
-      a.nc[k] = t.ncell[k];
-      a.ng[k] = t.ng[k];
-    }
-    a.tab = tabs[a.d];
-    a.final_pass = q == 2;
-    a.clear = clear;
-    const dim3 grid((a.Eout[0] * a.Eout[1] + 255) / 256, a.Eout[2]);
-    hipLaunchKernelGGL((k_m2m_pass<T, T>), grid, dim3(256), 0, st, static_cast<const T *>(ins[q]),
-                       static_cast<T *>(outs[q]), a);
-    PM_HIP(hipGetLastError());
-  }
+  M2MArgs a{};
+  a.f = f;
+  a.t = t;
+  a.reldx = f.dx[0] / t.dx[0];
+  a.clear = clear;
+  const T *src = static_cast<const T *>(from);
   T *dst = static_cast<T *>(to);
-  if (deposit) {
-    PGeom pg{};
-    for (int d = 0; d < 3; ++d) {
-      pg.ncell[d] = t.ncell[d];
-      pg.ngl[d] = t.ng[d];
-      pg.E[d] = t.E[d];
-    }
-    for (int d = 0; d < 3; ++d)
-      if (t.bc[d] != 0) {
-        hipLaunchKernelGGL(k_halo_add<T>, dim3(256), dim3(256), 0, st, dst, pg, d);
-        PM_HIP(hipGetLastError());
-      }
-  } else {
-    for (int d = 0; d < 3; ++d)
-      if (t.bc[d] != 0) {
-        hipLaunchKernelGGL(k_ghost_fill<T>, dim3(1024), dim3(256), 0, st, dst, t.E[0], t.E[1], t.E[2], d,
-                           t.ncell[d], t.ng[d], 3);
-        PM_HIP(hipGetLastError());
-      }
-  }
-  return 0;
+  const int e = deposit ? (ns == 6 ? m2m_down<T, 6>(a, src, dst, st) : m2m_down<T, 4>(a, src, dst, st))
+                        : (ns == 6 ? m2m_up<T, 6>(a, src, dst, st) : m2m_up<T, 4>(a, src, dst, st));
+  if (e > 0) return m2m_exact<T>(f, t, ns, from, to, clear, st);
+  if (e) return -1;
+  return m2m_periodic(t, deposit, dst, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -488,34 +811,14 @@ int m2m_exact(const MGeom &f, const MGeom &t, int ns, const void *from, void *to
     if (ns == 6) hipLaunchKernelGGL((k_m2m_deposit<T, 6>), grid, dim3(kTX), 0, st, src, dst, a);
     else hipLaunchKernelGGL((k_m2m_deposit<T, 4>), grid, dim3(kTX), 0, st, src, dst, a);
     PM_HIP(hipGetLastError());
-    // the ghost layers of periodic axes are added onto their images
-    // (:1380-1386, pmlib_mesh_map_ghost with incl_edges, op add)
-    PGeom pg{};
-    for (int d = 0; d < 3; ++d) {
-      pg.ncell[d] = t.ncell[d];
-      pg.ngl[d] = t.ng[d];
-      pg.E[d] = t.E[d];
-    }
-    for (int d = 0; d < 3; ++d)
-      if (t.bc[d] != 0) {
-        hipLaunchKernelGGL(k_halo_add<T>, dim3(256), dim3(256), 0, st, dst, pg, d);
-        PM_HIP(hipGetLastError());
-      }
   } else {
     const int64_t n = (int64_t)t.E[0] * t.E[1] * t.E[2];
     const int64_t blocks = std::min<int64_t>((n + 255) / 256, 65536);
     if (ns == 6) hipLaunchKernelGGL((k_m2m_interp<T, 6>), dim3(blocks), dim3(256), 0, st, src, dst, f, t, clear);
     else hipLaunchKernelGGL((k_m2m_interp<T, 4>), dim3(blocks), dim3(256), 0, st, src, dst, f, t, clear);
     PM_HIP(hipGetLastError());
-    // periodic ghosts copied from their images (:2057-2063, op replace)
-    for (int d = 0; d < 3; ++d)
-      if (t.bc[d] != 0) {
-        hipLaunchKernelGGL(k_ghost_fill<T>, dim3(1024), dim3(256), 0, st, dst, t.E[0], t.E[1], t.E[2], d,
-                           t.ncell[d], t.ng[d], 3);
-        PM_HIP(hipGetLastError());
-      }
   }
-  return 0;
+  return m2m_periodic(t, reldx <= 0.9999, dst, st);
 }
 
 int m2m_check(const pmgpu_geom *gf, const pmgpu_geom *gt, MGeom &f, MGeom &t) {
@@ -533,9 +836,7 @@ int m2m_check(const pmgpu_geom *gf, const pmgpu_geom *gt, MGeom &f, MGeom &t) {
 
 void m2m_release() {
   std::lock_guard<std::mutex> lock(g_m2m_mu);
-  void *bufs[] = {g_m2m.a, g_m2m.b, g_m2m.first, g_m2m.count, g_m2m.w};
-  for (void *b : bufs)
-    if (b) (void)hipFree(b);
+  if (g_m2m.a) (void)hipFree(g_m2m.a);
   g_m2m = M2MWS{};
 }
 }  // namespace pmgpu
