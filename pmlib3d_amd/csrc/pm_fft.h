@@ -105,6 +105,49 @@ template <int S, typename V> struct Dft<5, S, V> {
   }
 };
 
+// radix 2 q, q odd, as q radix-2 and two radix-q transforms: with r = 2 a + q b
+// (mod 2 q) the exponent r k / 2 q is a k / q + b k / 2, so no twiddles stand
+// between them and output k is that of k mod q and k mod 2
+template <int Q, int S, typename V> struct Dft2Q {
+  static __device__ __forceinline__ void run(V *v) {
+    V a[Q], b[Q];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      const V e = v[(2 * j) % (2 * Q)], o = v[(2 * j + Q) % (2 * Q)];
+      a[j] = cadd(e, o);
+      b[j] = csub(e, o);
+    }
+    Dft<Q, S, V>::run(a);
+    Dft<Q, S, V>::run(b);
+#pragma unroll
+    for (int k = 0; k < 2 * Q; ++k) v[k] = k % 2 == 0 ? a[k % Q] : b[k % Q];
+  }
+};
+template <int S, typename V> struct Dft<6, S, V> : Dft2Q<3, S, V> {};
+template <int S, typename V> struct Dft<10, S, V> : Dft2Q<5, S, V> {};
+
+// radix 12 = 3 x 4 in the same manner: r = 4 a + 3 b, r k / 12 = a k / 3 + b k / 4
+template <int S, typename V> struct Dft<12, S, V> {
+  static __device__ __forceinline__ void run(V *v) {
+    V t[3][4];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) t[a][b] = v[(4 * a + 3 * b) % 12];
+      Dft<4, S, V>::run(t[a]);
+    }
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2) {
+      V c[3] = {t[0][k2], t[1][k2], t[2][k2]};
+      Dft<3, S, V>::run(c);
+#pragma unroll
+      for (int k1 = 0; k1 < 3; ++k1) t[k1][k2] = c[k1];
+    }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) v[k] = t[k % 3][k % 4];
+  }
+};
+
 // Odd prime radix by direct summation; roots of unity come from the
 // length-L table (exp(-2 pi i m / R) = tw[m * L / R]).
 template <int R, int S, typename V> struct DftPrime {

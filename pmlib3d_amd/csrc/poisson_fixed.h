@@ -19,12 +19,13 @@ template <int NH, int VB> struct XLayout {
 // Line stride (complex words) of the register-resident kernels' LDS lines
 // for T columns per block (thread tid: column tid % T, position tid / T):
 // room for the padded line (i + i / 8), and g = 32 / T mod 32 words for
-// 8-byte FP32 complex (16 / T mod 16 for 16-byte FP64), g being the number
-// of positions a column has in one pass of the LDS (32 or 16 lanes), so the
-// T columns' runs of g consecutive positions tile the banks.
+// 8-byte FP32 complex (16 / T mod 16 for 16-byte FP64, at most 4), so the T
+// columns' runs of consecutive positions tile the banks.  (Transforms alone,
+// FP64 of 512 points: 2 columns 4 mod 16 0.62 ns per line on the whole chip,
+// 8 mod 16 0.66; 4 columns 4 mod 16 0.63, 8 mod 16 1.05, 0 mod 16 1.27.)
 template <int L, int VB, int T> constexpr int reg_line_stride() {
   const int mod = VB == 8 ? 32 : 16;
-  const int g = (mod / T) % mod;
+  const int g = VB == 16 && T == 2 ? 4 : (mod / T) % mod;
   int st = L + L / 8;
   while (st % mod != g) ++st;
   return st;
@@ -82,14 +83,14 @@ __global__ void __launch_bounds__(Geo<L>::P *T) k_strided_f(StridedArgs a, const
 template <typename R, int L, int T, int S, bool HALF>
 __device__ __forceinline__ void strided_r_body(const StridedArgs &a, const cplx_t<R> *tw, int64_t lt, int gx) {
   using V = cplx_t<R>;
-  constexpr int P = Geo<L>::P, ST = reg_line_stride<L, sizeof(V), T>(), E = L / P;
+  constexpr int K = strided_key<R>(L), P = Geo<K>::P, ST = reg_line_stride<L, sizeof(V), T>(), E = L / P;
   __shared__ V lds[T * ST];
   const int col0 = (int)(lt % gx) * T;
   const int64_t b = lt / gx;
   const int tid = threadIdx.x;
   const int col = tid % T, p = tid / T;
-  Twid<L, V> twd;
-  twid_load<L>(twd, p, tw + a.plan.tw_off);
+  Twid<K, V> twd;
+  twid_load<K>(twd, p, tw + a.plan.tw_off);
   const bool col_ok = col0 + col < a.ncols;
   const V *in = reinterpret_cast<const V *>(a.in) + b * a.bs_in + col0 + col;
   V *out = reinterpret_cast<V *>(a.out) + b * a.bs_out + col0 + col;
@@ -101,7 +102,7 @@ __device__ __forceinline__ void strided_r_body(const StridedArgs &a, const cplx_
   }
   // HALF: forward with the upper half of the rows zero, or inverse with only
   // the lower half wanted
-  fft_regs<L, S, V, HALF && (S < 0), HALF && (S > 0), 1>(x, lds + col * ST, p, twd);
+  fft_regs<K, S, V, HALF && (S < 0), HALF && (S > 0), 1>(x, lds + col * ST, p, twd);
   const R sc = (R)a.scale;
   if (col_ok) {
 #pragma unroll
@@ -112,7 +113,7 @@ __device__ __forceinline__ void strided_r_body(const StridedArgs &a, const cplx_
   }
 }
 template <typename R, int L, int T, int S, bool HALF>
-__global__ void __launch_bounds__(Geo<L>::P *T) k_strided_r(StridedArgs a, const cplx_t<R> *tw) {
+__global__ void __launch_bounds__((SGeo<R, L>::P * T)) k_strided_r(StridedArgs a, const cplx_t<R> *tw) {
   strided_r_body<R, L, T, S, HALF>(a, tw, xcd_tile(block_linear(), (int64_t)gridDim.x * gridDim.y * gridDim.z),
                                    gridDim.x);
 }
@@ -510,7 +511,7 @@ __device__ __forceinline__ double2 buf_load(__amdgpu_buffer_rsrc_t r, int voff, 
   return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
-// Velocity only.  Thread (col, p) of a block owns kx column kx0 + col (of TC
+// One output field, kernel 1.  Thread (col, p) of a block owns kx column kx0 + col (of TC
 // consecutive ones) and the z rows p + P m of all three components: its loads
 // and stores are whole cache lines across the block's lanes (consecutive
 // columns, components interleaved), the first and last FFT stages run on the
@@ -521,10 +522,22 @@ __device__ __forceinline__ double2 buf_load(__amdgpu_buffer_rsrc_t r, int voff, 
 // HALF (free-space z, Mz = L / 2): rows >= L / 2 are zero on the way in and
 // not wanted on the way out, so the first forward and the last inverse stage
 // skip them.
-template <typename R, int L, int TC, bool ALLPER, bool HALF>
-__global__ void __launch_bounds__(Geo<L>::P *TC) k_z3_r(ZArgs a, const cplx_t<R> *tw_all) {
+// FIELD: the velocity in place (kVel; kVelFiltered: with every axis periodic
+// the spectral G carries the filter zeta as well when the vorticity is
+// filtered, poisson/pmlib_poisson_solve.f:339-349), or psi-hat = G w-hat or
+// zeta w-hat [+ reprojection] into their own spectra (:767-872).  A solve with
+// more outputs than the velocity launches the others first: a forward
+// transform more for each, but a kernel that forms them all keeps its spectra
+// in registers or LDS at one wavefront per SIMD (256^3 FP64 velocity and
+// vorticity 3.25 ms, in two launches 2.30; 64^3 FP64 velocity and psi 58, 47 us).
+// (The vorticity in FP64 is held to two wavefronts per SIMD at 4 to 20 spilled
+// registers: 2.06 -> 1.43 ms.)
+constexpr int kVel = 0, kPsi = 1, kVort = 2, kVelFiltered = 3;
+template <typename R, int L, int TC, bool ALLPER, bool HALF, int FIELD>
+__global__ void __launch_bounds__(RGeo<L>::P *TC, sizeof(R) == 8 && FIELD == kVort ? 2 : 1)
+    k_z3_r(ZArgs a, const cplx_t<R> *tw_all) {
   using V = cplx_t<R>;
-  constexpr int P = Geo<L>::P, E = L / P;
+  constexpr int K = reg_key(L), P = Geo<K>::P, E = L / P;
   // line stride between the block's columns for the i + i / 8 padding
   constexpr int ST = reg_line_stride<L, sizeof(V), TC>();
   __shared__ V lds[TC * ST];
@@ -533,8 +546,8 @@ __global__ void __launch_bounds__(Geo<L>::P *TC) k_z3_r(ZArgs a, const cplx_t<R>
   const int kx0 = (int)(lt % gridDim.x) * TC, ky = (int)(lt / gridDim.x);
   const int tid = threadIdx.x;
   const int col = tid % TC, p = tid / TC;
-  Twid<L, V> twd;
-  twid_load<L>(twd, p, tw);
+  Twid<K, V> twd;
+  twid_load<K>(twd, p, tw);
   const int kx = kx0 + col;
   const bool col_ok = kx < a.Hx;
   // this block's tile: rows [0, Mz) of columns kx0 .. kx0 + TC - 1 (3 words each)
@@ -555,14 +568,16 @@ __global__ void __launch_bounds__(Geo<L>::P *TC) k_z3_r(ZArgs a, const cplx_t<R>
   }
   V *line = lds + col * ST;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) fft_regs<L, -1, V, HALF, false, 1>(w[c], line, p, twd);
+  for (int c = 0; c < 3; ++c) fft_regs<K, -1, V, HALF, false, 1>(w[c], line, p, twd);
   // u-hat = G 2 pi i (k x w-hat); Nyquist wavenumbers drop out (Hermitian
   // projection of the real inverse); the 1 / L of the inverse transform
   // rides on the same factor
   const R ki = wavenumber<R>(kx, a.Lx, a.dk[0], a.ksmp[0]);
   const R kj = wavenumber<R>(ky, a.Ly, a.dk[1], a.ksmp[1]);
-  const R kx_ = (2 * kx == a.Lx) ? (R)0 : ki, ky_ = (2 * ky == a.Ly) ? (R)0 : kj;
+  const bool nx = 2 * kx == a.Lx, ny = 2 * ky == a.Ly;
+  const R kx_ = nx ? (R)0 : ki, ky_ = ny ? (R)0 : kj;
   const int kyf = ky <= a.Ly - ky ? ky : a.Ly - ky;
+  const R pi = (R)3.14159265358979323846, inv_l = (R)1 / (R)L;
   const R twopi = (R)6.28318530717958647692 / (R)L;
   // G-hat of the thread's rows, all loads issued before any is used (a
   // column past Hx reads column 0 and is masked)
@@ -581,174 +596,63 @@ __global__ void __launch_bounds__(Geo<L>::P *TC) k_z3_r(ZArgs a, const cplx_t<R>
   for (int m = 0; m < E; ++m) {
     const int n = p + P * m;
     const R kk = wavenumber<R>(n, L, a.dk[2], a.ksmp[2]);
-    R g;
+    R zeta = (R)1, g;
+    if (FIELD == kVort || FIELD == kVelFiltered || (FIELD == kPsi && ALLPER && a.want_vort))
+      zeta = zeta_filter<R>(a.order, (R)a.eps2pi * sqrt(ki * ki + kj * kj + kk * kk));
     if constexpr (ALLPER) {
       const R kmag = ki * ki + kj * kj + kk * kk;
-      const R pi = (R)3.14159265358979323846;
-      g = kmag > (R)0 ? (R)1 / ((R)4 * (pi * pi) * kmag) : (R)0;
+      g = kmag > (R)0 ? zeta / ((R)4 * (pi * pi) * kmag) : (R)0;
     } else {
       g = col_ok ? gv[m] * (R)a.h3 : (R)0;
     }
-    const R kz_ = (2 * n == L) ? (R)0 : kk;
+    const bool nz = 2 * n == L;
     const V w0 = w[0][m], w1 = w[1][m], w2 = w[2][m];
-    const V c0 = csub(cscale(w2, ky_), cscale(w1, kz_));
-    const V c1 = csub(cscale(w0, kz_), cscale(w2, kx_));
-    const V c2 = csub(cscale(w1, kx_), cscale(w0, ky_));
-    const R f = g * twopi;
-    w[0][m] = cmake<V>(-c0.y * f, c0.x * f);
-    w[1][m] = cmake<V>(-c1.y * f, c1.x * f);
-    w[2][m] = cmake<V>(-c2.y * f, c2.x * f);
+    if constexpr (FIELD == kVel || FIELD == kVelFiltered) {
+      const R kz_ = nz ? (R)0 : kk;
+      const V c0 = csub(cscale(w2, ky_), cscale(w1, kz_));
+      const V c1 = csub(cscale(w0, kz_), cscale(w2, kx_));
+      const V c2 = csub(cscale(w1, kx_), cscale(w0, ky_));
+      const R f = g * twopi;
+      w[0][m] = cmake<V>(-c0.y * f, c0.x * f);
+      w[1][m] = cmake<V>(-c1.y * f, c1.x * f);
+      w[2][m] = cmake<V>(-c2.y * f, c2.x * f);
+    } else if constexpr (FIELD == kPsi) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) w[c][m] = cscale(w[c][m], g * inv_l);
+    } else {
+      // reprojection: -4 pi^2 G k_c sum_d k_d w_d over the pairs (c, d) of
+      // equal Nyquist parity (:861-872)
+      const R kd[3] = {ki, kj, kk};
+      const bool nd[3] = {nx, ny, nz};
+      const R f = a.reproj ? -(R)4 * (pi * pi) * g * inv_l : (R)0;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const V wc = c == 0 ? w0 : (c == 1 ? w1 : w2);
+        V q = cscale(wc, zeta * inv_l);
+        if (a.reproj) {
+          V acc = cmake<V>(0, 0);
+          if (nd[0] == nd[c]) acc = cadd(acc, cscale(w0, ki));
+          if (nd[1] == nd[c]) acc = cadd(acc, cscale(w1, kj));
+          if (nd[2] == nd[c]) acc = cadd(acc, cscale(w2, kk));
+          q = cadd(q, cscale(acc, f * kd[c]));
+        }
+        w[c][m] = q;
+      }
+    }
   }
 #pragma unroll
-  for (int c = 0; c < 3; ++c) fft_regs<L, 1, V, false, HALF, 1>(w[c], line, p, twd);
+  for (int c = 0; c < 3; ++c) fft_regs<K, 1, V, false, HALF, 1>(w[c], line, p, twd);
   // Stores are plain global stores: buffer-resource stores of these
   // 8-byte-aligned records, which the compiler merges into 16-byte stores
   // across components, have returned corrupted first components.
   if (col_ok) {
-    V *dst = base + (int64_t)p * a.rs + col * 3;
+    V *out = FIELD == kPsi ? reinterpret_cast<V *>(a.Bpsi) : reinterpret_cast<V *>(FIELD == kVort ? a.Bvort : a.B);
+    V *dst = out + (int64_t)ky * a.kys + (int64_t)kx0 * 3 + (int64_t)p * a.rs + col * 3;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       if (HALF ? m < E / 2 : p + P * m < a.Mz) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) dst[(int64_t)P * m * a.rs + c] = w[c][m];
-      }
-    }
-  }
-}
-
-// Full-output form of k_z3_r: velocity plus the stream function and/or the
-// filtered (and optionally reprojected) vorticity, kernel 1.  The three
-// forward spectra stay in registers; each requested field is formed from
-// them in registers, transformed back (one component at a time through the
-// same LDS line) and stored, velocity in place, psi-hat and zeta-hat into
-// their own spectra (poisson/pmlib_poisson_solve.f:767-872: psi = G w-hat,
-// vort = zeta w-hat [+ reprojection]).  With every axis periodic the
-// spectral G carries the filter zeta as well when the vorticity is filtered
-// (:339-349).
-// SL: the forward spectra wait in LDS (each thread reads back only the words
-// it wrote, so no barrier) instead of registers, for FP64's register budget.
-template <typename R, int L, int TC, bool ALLPER, bool HALF, bool SL>
-__global__ void __launch_bounds__(Geo<L>::P *TC) k_z3_rx(ZArgs a, const cplx_t<R> *tw_all) {
-  using V = cplx_t<R>;
-  constexpr int P = Geo<L>::P, E = L / P;
-  constexpr int ST = reg_line_stride<L, sizeof(V), TC>();
-  __shared__ V lds[TC * ST];
-  __shared__ V spec[SL ? TC * 3 * L : 1];
-  const V *tw = tw_all + a.plan.tw_off;
-  const int64_t lt = xcd_tile(block_linear(), (int64_t)gridDim.x * gridDim.y);
-  const int kx0 = (int)(lt % gridDim.x) * TC, ky = (int)(lt / gridDim.x);
-  const int tid = threadIdx.x;
-  const int col = tid % TC, p = tid / TC;
-  Twid<L, V> twd;
-  twid_load<L>(twd, p, tw);
-  const int kx = kx0 + col;
-  const bool col_ok = kx < a.Hx;
-  const int64_t toff = (int64_t)ky * a.kys + (int64_t)kx0 * 3;
-  V *base = reinterpret_cast<V *>(a.B) + toff;
-  const int64_t rsb = a.rs * (int64_t)sizeof(V);
-  const int ncols_here = a.Hx - kx0 < TC ? a.Hx - kx0 : TC;
-  const uint32_t extent = (uint32_t)((a.Mz - 1) * rsb + (int64_t)ncols_here * 3 * sizeof(V));
-  const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(base, extent);
-  const int voff = (int)(p * rsb) + col * 3 * (int)sizeof(V);
-  V w[3][E];
-#pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const bool ok = col_ok && (HALF ? m < E / 2 : p + P * m < a.Mz);
-    const int soff = (int)((int64_t)P * m * rsb);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      w[c][m] = ok ? buf_load(rsrc, voff + c * (int)sizeof(V), soff, V{}) : cmake<V>(0, 0);
-  }
-  V *line = lds + col * ST;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) fft_regs<L, -1, V, HALF, false, 1>(w[c], line, p, twd);
-  V *sp = spec + (SL ? col * 3 * L + p : 0);   // word (c, m) at sp[(c E + m) P]
-  if constexpr (SL) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int m = 0; m < E; ++m) sp[(c * E + m) * P] = w[c][m];
-  }
-  auto spw = [&](int c, int m) -> V { return SL ? sp[(c * E + m) * P] : w[c][m]; };
-  const R ki = wavenumber<R>(kx, a.Lx, a.dk[0], a.ksmp[0]);
-  const R kj = wavenumber<R>(ky, a.Ly, a.dk[1], a.ksmp[1]);
-  const bool nx = (2 * kx == a.Lx), ny = (2 * ky == a.Ly);
-  const R kx_ = nx ? (R)0 : ki, ky_ = ny ? (R)0 : kj;
-  const int kyf = ky <= a.Ly - ky ? ky : a.Ly - ky;
-  const R pi = (R)3.14159265358979323846;
-  const R twopi = (R)6.28318530717958647692;
-  // per row: G h^3 (with zeta when all axes are periodic and the vorticity
-  // is filtered) and zeta
-  R gz[E], zt[E];
-  {
-    const R *G = reinterpret_cast<const R *>(a.Ghat) + (int64_t)kyf * a.Hx + (col_ok ? kx : 0);
-    const int64_t gzs = (int64_t)a.Hy * a.Hx;
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-      const int n = p + P * m;
-      const R kk = wavenumber<R>(n, L, a.dk[2], a.ksmp[2]);
-      zt[m] = a.want_vort ? zeta_filter<R>(a.order, (R)a.eps2pi * sqrt(ki * ki + kj * kj + kk * kk)) : (R)1;
-      if constexpr (ALLPER) {
-        const R kmag = ki * ki + kj * kj + kk * kk;
-        gz[m] = kmag > (R)0 ? zt[m] / ((R)4 * (pi * pi) * kmag) : (R)0;
-      } else {
-        const int kzf = n <= L - n ? n : L - n;
-        gz[m] = col_ok ? G[kzf * gzs] * (R)a.h3 : (R)0;
-      }
-    }
-  }
-  const R scale = (R)1 / (R)L;
-  const int nkind = 1 + (a.want_psi ? 1 : 0) + (a.want_vort ? 1 : 0);
-  // one output component at a time: only its E words are live beside the
-  // three forward spectra
-#pragma unroll 1
-  for (int kd = 0; kd < nkind; ++kd) {
-    const int kind = kd == 0 ? 0 : ((kd == 1 && a.want_psi) ? 1 : 2);
-    V *out = (kind == 0 ? reinterpret_cast<V *>(a.B)
-                        : (kind == 1 ? reinterpret_cast<V *>(a.Bpsi) : reinterpret_cast<V *>(a.Bvort))) + toff;
-#pragma unroll 1
-    for (int c = 0; c < 3; ++c) {
-      V r[E];
-#pragma unroll
-      for (int m = 0; m < E; ++m) {
-        const int n = p + P * m;
-        const R kk = wavenumber<R>(n, L, a.dk[2], a.ksmp[2]);
-        const bool nz = (2 * n == L);
-        const V w0 = spw(0, m), w1 = spw(1, m), w2 = spw(2, m);
-        const V wc = c == 0 ? w0 : (c == 1 ? w1 : w2);
-        if (kind == 0) {
-          // u-hat = G 2 pi i (k x w-hat), Nyquist wavenumbers dropped
-          const R kz_ = nz ? (R)0 : kk;
-          V cr;
-          if (c == 0) cr = csub(cscale(w2, ky_), cscale(w1, kz_));
-          else if (c == 1) cr = csub(cscale(w0, kz_), cscale(w2, kx_));
-          else cr = csub(cscale(w1, kx_), cscale(w0, ky_));
-          const R f = gz[m] * twopi;
-          r[m] = cmake<V>(-cr.y * f, cr.x * f);
-        } else if (kind == 1) {
-          r[m] = cscale(wc, gz[m]);
-        } else {
-          V q = cscale(wc, zt[m]);
-          if (a.reproj) {
-            // -4 pi^2 G k_c sum_d k_d w_d over the pairs (c, d) of equal
-            // Nyquist parity (:861-872)
-            const bool nc = c == 0 ? nx : (c == 1 ? ny : nz);
-            const R kc = c == 0 ? ki : (c == 1 ? kj : kk);
-            V acc = cmake<V>(0, 0);
-            if (nx == nc) acc = cadd(acc, cscale(w0, ki));
-            if (ny == nc) acc = cadd(acc, cscale(w1, kj));
-            if (nz == nc) acc = cadd(acc, cscale(w2, kk));
-            q = cadd(q, cscale(acc, -(R)4 * (pi * pi) * gz[m] * kc));
-          }
-          r[m] = q;
-        }
-      }
-      fft_regs<L, 1, V, false, HALF, 1>(r, line, p, twd);
-      if (col_ok) {
-        V *dst = out + (int64_t)p * a.rs + col * 3 + c;
-#pragma unroll
-        for (int m = 0; m < E; ++m)
-          if (HALF ? m < E / 2 : p + P * m < a.Mz) dst[(int64_t)P * m * a.rs] = cscale(r[m], scale);
       }
     }
   }
@@ -836,15 +740,15 @@ __global__ void __launch_bounds__(Geo<L>::P *T) k_z1_f(ZArgs a, const cplx_t<R> 
 template <typename R, int L, int TC, bool ALLPER, bool HALF>
 __device__ __forceinline__ void z1_r_body(const ZArgs &a, const cplx_t<R> *tw_all, int64_t lt, int gx) {
   using V = cplx_t<R>;
-  constexpr int P = Geo<L>::P, E = L / P;
+  constexpr int K = reg_key(L), P = Geo<K>::P, E = L / P;
   constexpr int ST = reg_line_stride<L, sizeof(V), TC>();
   __shared__ V lds[TC * ST];
   const V *tw = tw_all + a.plan.tw_off;
   const int kx0 = (int)(lt % gx) * TC, ky = (int)(lt / gx);
   const int tid = threadIdx.x;
   const int col = tid % TC, p = tid / TC;
-  Twid<L, V> twd;
-  twid_load<L>(twd, p, tw);
+  Twid<K, V> twd;
+  twid_load<K>(twd, p, tw);
   const int kx = kx0 + col;
   const bool col_ok = kx < a.Hx;
   V *base = reinterpret_cast<V *>(a.B) + (int64_t)ky * a.kys + kx0;
@@ -860,7 +764,7 @@ __device__ __forceinline__ void z1_r_body(const ZArgs &a, const cplx_t<R> *tw_al
     w[m] = ok ? buf_load(rsrc, voff, (int)((int64_t)P * m * rsb), V{}) : cmake<V>(0, 0);
   }
   V *line = lds + col * ST;
-  fft_regs<L, -1, V, HALF, false, 1>(w, line, p, twd);
+  fft_regs<K, -1, V, HALF, false, 1>(w, line, p, twd);
   const int kyf = ky <= a.Ly - ky ? ky : a.Ly - ky;
   if constexpr (ALLPER) {
     const R ki = wavenumber<R>(kx, a.Lx, a.dk[0], a.ksmp[0]);
@@ -886,7 +790,7 @@ __device__ __forceinline__ void z1_r_body(const ZArgs &a, const cplx_t<R> *tw_al
 #pragma unroll
     for (int m = 0; m < E; ++m) w[m] = cscale(w[m], gv[m] * (R)a.h3);
   }
-  fft_regs<L, 1, V, false, HALF, 1>(w, line, p, twd);
+  fft_regs<K, 1, V, false, HALF, 1>(w, line, p, twd);
   const R scale = (R)1 / (R)L;
   if (col_ok) {
     V *dst = base + (int64_t)p * a.rs + col;
@@ -896,7 +800,7 @@ __device__ __forceinline__ void z1_r_body(const ZArgs &a, const cplx_t<R> *tw_al
   }
 }
 template <typename R, int L, int TC, bool ALLPER, bool HALF>
-__global__ void __launch_bounds__(Geo<L>::P *TC) k_z1_r(ZArgs a, const cplx_t<R> *tw_all) {
+__global__ void __launch_bounds__(RGeo<L>::P *TC) k_z1_r(ZArgs a, const cplx_t<R> *tw_all) {
   z1_r_body<R, L, TC, ALLPER, HALF>(a, tw_all, xcd_tile(block_linear(), (int64_t)gridDim.x * gridDim.y), gridDim.x);
 }
 
@@ -932,7 +836,7 @@ __global__ void __launch_bounds__(Geo<L>::P *T)
   strided_f_body<R, L, T, S>(g.a, reinterpret_cast<const cplx_t<R> *>(g.tw), g.lt, g.gx);
 }
 template <typename R, int L, int T, int S, bool HALF>
-__global__ void __launch_bounds__(Geo<L>::P *T)
+__global__ void __launch_bounds__((SGeo<R, L>::P * T))
     kg_strided_r(const GrpEntry<StridedArgs> *__restrict__ t, int n, int64_t nb) {
   const GrpTile<StridedArgs> g = grp_tile(t, n, nb);
   strided_r_body<R, L, T, S, HALF>(g.a, reinterpret_cast<const cplx_t<R> *>(g.tw), g.lt, g.gx);
@@ -955,7 +859,7 @@ __global__ void __launch_bounds__(Geo<L>::P *T) kg_z1_f(const GrpEntry<ZArgs> *_
   z1_f_body<R, L, T>(g.a, reinterpret_cast<const cplx_t<R> *>(g.tw), g.lt, g.gx);
 }
 template <typename R, int L, int TC, bool ALLPER, bool HALF>
-__global__ void __launch_bounds__(Geo<L>::P *TC) kg_z1_r(const GrpEntry<ZArgs> *__restrict__ t, int n, int64_t nb) {
+__global__ void __launch_bounds__(RGeo<L>::P *TC) kg_z1_r(const GrpEntry<ZArgs> *__restrict__ t, int n, int64_t nb) {
   const GrpTile<ZArgs> g = grp_tile(t, n, nb);
   z1_r_body<R, L, TC, ALLPER, HALF>(g.a, reinterpret_cast<const cplx_t<R> *>(g.tw), g.lt, g.gx);
 }

@@ -34,20 +34,20 @@ template <typename R, int NH, int NC> constexpr int tile_lines() {
 
 template <typename R, int L>
 int strided_L(int S, StridedArgs a, int nb_y, int nb_z, const cplx_t<R> *tw, hipStream_t st) {
-  if constexpr (regs_ok<L>()) {
+  if constexpr (regs_ok<strided_key<R>(L)>()) {
     if (a.kernel == 0) {
       constexpr int T = tile_cols<R, L>();
       a.T = T;
       dim3 grid((a.ncols + T - 1) / T, nb_y, nb_z);
-      const bool half = (L / Geo<L>::P) % 2 == 0 && (S < 0 ? 2 * a.nin == L : 2 * a.nout == L);
+      const bool half = (L / SGeo<R, L>::P) % 2 == 0 && (S < 0 ? 2 * a.nin == L : 2 * a.nout == L);
       if (S < 0 && half)
-        hipLaunchKernelGGL((k_strided_r<R, L, T, -1, true>), grid, dim3(Geo<L>::P * T), 0, st, a, tw);
+        hipLaunchKernelGGL((k_strided_r<R, L, T, -1, true>), grid, dim3(SGeo<R, L>::P * T), 0, st, a, tw);
       else if (S < 0)
-        hipLaunchKernelGGL((k_strided_r<R, L, T, -1, false>), grid, dim3(Geo<L>::P * T), 0, st, a, tw);
+        hipLaunchKernelGGL((k_strided_r<R, L, T, -1, false>), grid, dim3(SGeo<R, L>::P * T), 0, st, a, tw);
       else if (half)
-        hipLaunchKernelGGL((k_strided_r<R, L, T, 1, true>), grid, dim3(Geo<L>::P * T), 0, st, a, tw);
+        hipLaunchKernelGGL((k_strided_r<R, L, T, 1, true>), grid, dim3(SGeo<R, L>::P * T), 0, st, a, tw);
       else
-        hipLaunchKernelGGL((k_strided_r<R, L, T, 1, false>), grid, dim3(Geo<L>::P * T), 0, st, a, tw);
+        hipLaunchKernelGGL((k_strided_r<R, L, T, 1, false>), grid, dim3(SGeo<R, L>::P * T), 0, st, a, tw);
       return hipGetLastError() == hipSuccess ? 1 : -1;
     }
   }
@@ -76,65 +76,49 @@ template <typename R, int L, int TC> int z_tc(ZArgs a, int Ly, const cplx_t<R> *
   return hipGetLastError() == hipSuccess ? 1 : -1;
 }
 
-// register-resident velocity z pass with TC columns per block
-template <typename R, int L, int TC> int zr_T(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
-  if constexpr (!regs_ok<L>() || TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
-                Geo<L>::P * TC > 1024) {
+// register-resident z pass of one field with TC columns per block
+template <typename R, int L, int TC, int FIELD> int zr_T(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
+  if constexpr (!regs_ok<reg_key(L)>() ||
+                TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
+                RGeo<L>::P * TC > 1024) {
     return 0;
   } else {
     // buffer offsets of the tile are 31-bit
     if ((double)a.Mz * (double)a.rs * sizeof(cplx_t<R>) >= 2147483647.0) return 0;
-    dim3 grid((a.Hx + TC - 1) / TC, Ly);
+    dim3 grid((a.Hx + TC - 1) / TC, Ly), block(RGeo<L>::P * TC);
     if (a.allper)
-      hipLaunchKernelGGL((k_z3_r<R, L, TC, true, false>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
-    else if (2 * a.Mz == L && (L / Geo<L>::P) % 2 == 0)
-      hipLaunchKernelGGL((k_z3_r<R, L, TC, false, true>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
+      hipLaunchKernelGGL((k_z3_r<R, L, TC, true, false, FIELD>), grid, block, 0, st, a, tw);
+    else if constexpr (FIELD == kVelFiltered)
+      return 0;
+    else if (2 * a.Mz == L && (L / RGeo<L>::P) % 2 == 0)
+      hipLaunchKernelGGL((k_z3_r<R, L, TC, false, true, FIELD>), grid, block, 0, st, a, tw);
     else
-      hipLaunchKernelGGL((k_z3_r<R, L, TC, false, false>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
+      hipLaunchKernelGGL((k_z3_r<R, L, TC, false, false, FIELD>), grid, block, 0, st, a, tw);
     return hipGetLastError() == hipSuccess ? 1 : -1;
   }
-}
-// register-resident full-output z pass (psi and/or filtered vorticity); SL
-// keeps the forward spectra in LDS
-template <typename R, int L, int TC, bool SL>
-int zrx_T(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
-  constexpr int lds_bytes = (TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() + (SL ? TC * 3 * L : 0)) *
-                            (int)sizeof(cplx_t<R>);
-  if constexpr (!regs_ok<L>() || lds_bytes > kLdsBudget || Geo<L>::P * TC > 1024) {
-    return 0;
-  } else {
-    if ((double)a.Mz * (double)a.rs * sizeof(cplx_t<R>) >= 2147483647.0) return 0;
-    dim3 grid((a.Hx + TC - 1) / TC, Ly);
-    if (a.allper)
-      hipLaunchKernelGGL((k_z3_rx<R, L, TC, true, false, SL>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
-    else if (2 * a.Mz == L && (L / Geo<L>::P) % 2 == 0)
-      hipLaunchKernelGGL((k_z3_rx<R, L, TC, false, true, SL>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
-    else
-      hipLaunchKernelGGL((k_z3_rx<R, L, TC, false, false, SL>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
-    return hipGetLastError() == hipSuccess ? 1 : -1;
-  }
-}
-template <typename R, int L> int zrx_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
-  // FP32: spectra in registers, 4 columns per block; FP64: spectra in LDS
-  // (the register form runs at one wave per SIMD), 2 or 1 columns as LDS allows
-  static const int form = [] {
-    const char *e = getenv("PMGPU_ZRX");
-    return e ? atoi(e) : -1;
-  }();
-  const bool sl = form >= 0 ? form == 1 : sizeof(R) == 8;
-  if (!sl) return zrx_T<R, L, 4, false>(a, Ly, tw, st);
-  const int r = zrx_T<R, L, 2, true>(a, Ly, tw, st);
-  return r != 0 ? r : zrx_T<R, L, 1, true>(a, Ly, tw, st);
 }
 
 template <typename R, int L> int zr_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
   const int want = a.tune_tc > 0 ? a.tune_tc : 4;
   switch (want) {
-    case 2: return zr_T<R, L, 2>(a, Ly, tw, st);
-    case 4: return zr_T<R, L, 4>(a, Ly, tw, st);
-    case 8: return zr_T<R, L, 8>(a, Ly, tw, st);
+    case 2: return zr_T<R, L, 2, kVel>(a, Ly, tw, st);
+    case 4: return zr_T<R, L, 4, kVel>(a, Ly, tw, st);
+    case 8: return zr_T<R, L, 8, kVel>(a, Ly, tw, st);
     default: return 0;
   }
+}
+// the velocity (last: in place) with the stream function and/or the vorticity
+template <typename R, int L> int zrx_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
+  if (a.want_psi) {
+    const int r = zr_T<R, L, 4, kPsi>(a, Ly, tw, st);
+    if (r != 1) return r;
+  }
+  if (a.want_vort) {
+    const int r = zr_T<R, L, 4, kVort>(a, Ly, tw, st);
+    if (r != 1) return r;
+    if (a.allper) return zr_T<R, L, 4, kVelFiltered>(a, Ly, tw, st);
+  }
+  return zr_T<R, L, 4, kVel>(a, Ly, tw, st);
 }
 
 template <typename R, int L> int z_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
@@ -214,18 +198,19 @@ template <typename R, int L, int T> int z1_T(ZArgs a, int Ly, const cplx_t<R> *t
 }
 // register-resident scalar z pass, TC columns per block
 template <typename R, int L, int TC> int z1r_T(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
-  if constexpr (!regs_ok<L>() || TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
-                Geo<L>::P * TC > 1024) {
+  if constexpr (!regs_ok<reg_key(L)>() ||
+                TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
+                RGeo<L>::P * TC > 1024) {
     return 0;
   } else {
     if ((double)a.Mz * (double)a.rs * sizeof(cplx_t<R>) >= 2147483647.0) return 0;  // 31-bit buffer offsets
     dim3 grid((a.Hx + TC - 1) / TC, Ly);
     if (a.allper)
-      hipLaunchKernelGGL((k_z1_r<R, L, TC, true, false>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
-    else if (2 * a.Mz == L && (L / Geo<L>::P) % 2 == 0)
-      hipLaunchKernelGGL((k_z1_r<R, L, TC, false, true>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
+      hipLaunchKernelGGL((k_z1_r<R, L, TC, true, false>), grid, dim3(RGeo<L>::P * TC), 0, st, a, tw);
+    else if (2 * a.Mz == L && (L / RGeo<L>::P) % 2 == 0)
+      hipLaunchKernelGGL((k_z1_r<R, L, TC, false, true>), grid, dim3(RGeo<L>::P * TC), 0, st, a, tw);
     else
-      hipLaunchKernelGGL((k_z1_r<R, L, TC, false, false>), grid, dim3(Geo<L>::P * TC), 0, st, a, tw);
+      hipLaunchKernelGGL((k_z1_r<R, L, TC, false, false>), grid, dim3(RGeo<L>::P * TC), 0, st, a, tw);
     return hipGetLastError() == hipSuccess ? 1 : -1;
   }
 }
@@ -234,8 +219,9 @@ template <typename R, int L, int T> constexpr bool z1_fits() {
   return T * Geo<L>::ST * (int)sizeof(cplx_t<R>) <= kLdsBudget && Geo<L>::P * T <= 1024;
 }
 template <typename R, int L, int TC> constexpr bool z1r_fits() {
-  return regs_ok<L>() && TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) <= kLdsBudget &&
-         Geo<L>::P * TC <= 1024;
+  return regs_ok<reg_key(L)>() &&
+         TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) <= kLdsBudget &&
+         RGeo<L>::P * TC <= 1024;
 }
 template <typename R, int L> int z1_avail(int T) {
   switch (T) {
@@ -281,17 +267,17 @@ template <typename R, int NH> int grp_xinv_L(const GrpEntry<XInvArgs> *t, int n,
 template <typename R, int L>
 int grp_strided_L(int S, int kernel, bool half, const GrpEntry<StridedArgs> *t, int n, int64_t nb, hipStream_t st) {
   constexpr int T = tile_cols<R, L>();
-  const dim3 grid((unsigned)nb), block(Geo<L>::P * T);
-  if constexpr (regs_ok<L>()) {
+  const dim3 grid((unsigned)nb), block(Geo<L>::P * T), rblock(SGeo<R, L>::P * T);
+  if constexpr (regs_ok<strided_key<R>(L)>()) {
     if (kernel == 0) {
       if (S < 0 && half)
-        hipLaunchKernelGGL((kg_strided_r<R, L, T, -1, true>), grid, block, 0, st, t, n, nb);
+        hipLaunchKernelGGL((kg_strided_r<R, L, T, -1, true>), grid, rblock, 0, st, t, n, nb);
       else if (S < 0)
-        hipLaunchKernelGGL((kg_strided_r<R, L, T, -1, false>), grid, block, 0, st, t, n, nb);
+        hipLaunchKernelGGL((kg_strided_r<R, L, T, -1, false>), grid, rblock, 0, st, t, n, nb);
       else if (half)
-        hipLaunchKernelGGL((kg_strided_r<R, L, T, 1, true>), grid, block, 0, st, t, n, nb);
+        hipLaunchKernelGGL((kg_strided_r<R, L, T, 1, true>), grid, rblock, 0, st, t, n, nb);
       else
-        hipLaunchKernelGGL((kg_strided_r<R, L, T, 1, false>), grid, block, 0, st, t, n, nb);
+        hipLaunchKernelGGL((kg_strided_r<R, L, T, 1, false>), grid, rblock, 0, st, t, n, nb);
       return hipGetLastError() == hipSuccess ? 1 : -1;
     }
   }
@@ -313,11 +299,12 @@ int grp_z1_T(const GrpEntry<ZArgs> *t, int n, int64_t nb, hipStream_t st) {
 }
 template <typename R, int L, int TC>
 int grp_z1r_T(bool allper, bool half, const GrpEntry<ZArgs> *t, int n, int64_t nb, hipStream_t st) {
-  if constexpr (!regs_ok<L>() || TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
-                Geo<L>::P * TC > 1024) {
+  if constexpr (!regs_ok<reg_key(L)>() ||
+                TC * reg_line_stride<L, sizeof(cplx_t<R>), TC>() * (int)sizeof(cplx_t<R>) > kLdsBudget ||
+                RGeo<L>::P * TC > 1024) {
     return 0;
   } else {
-    const dim3 grid((unsigned)nb), block(Geo<L>::P * TC);
+    const dim3 grid((unsigned)nb), block(RGeo<L>::P * TC);
     if (allper)
       hipLaunchKernelGGL((kg_z1_r<R, L, TC, true, false>), grid, block, 0, st, t, n, nb);
     else if (half)
@@ -346,7 +333,7 @@ int grp_z1_L(int T, bool allper, bool half, const GrpEntry<ZArgs> *t, int n, int
 template <typename R, int L> const FxOps<R> *fx_ops() {
   static const FxOps<R> ops{&strided_L<R, L>,      &z_L<R, L>,          &xfwd_L<R, L>,       &xinv_L<R, L>,
                             &z1_L<R, L>,           &z1_avail<R, L>,     tile_lines<R, L, 1>(), tile_cols<R, L>(),
-                            (L / Geo<L>::P) % 2 == 0 ? 1 : 0, &grp_xfwd_L<R, L>, &grp_xinv_L<R, L>,
+                            (L / RGeo<L>::P) % 2 == 0 ? 1 : 0, &grp_xfwd_L<R, L>, &grp_xinv_L<R, L>,
                             &grp_strided_L<R, L>, &grp_z1_L<R, L>};
   return &ops;
 }
