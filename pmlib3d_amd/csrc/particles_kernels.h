@@ -9,6 +9,8 @@
 // contiguous range of records), in a fixed order.  No atomics touch the
 // mesh, so the result is deterministic run to run.
 #pragma once
+#include <type_traits>
+
 #include "pm_common.h"
 
 namespace pmgpu {
@@ -731,13 +733,48 @@ template <typename T> __global__ void k_halo_add(T *m, PGeom g, int d) {
 // compensated FP32 sum).
 // Stencil weights and indices live in registers (the stencil width is a
 // template parameter).
+//
+// What bounds it: the L1, which takes about 16 cycles per load instruction of a
+// wavefront, however narrow.  A stencil row's ns nodes lie side by side, so a
+// row is read as the one run of 3 ns words they make (M'4: 6 dwordx4 in FP64, 3
+// in FP32) instead of node by node (8 and 4 loads).  us before and now: 128^3 FP64
+// M'4 periodic 191, 149, free 189, 155; M6* free 572, 475; FP32 M'4 92, 75 and
+// 104, 97; M6* free 322, 283; 384^3 FP32 2270, 2020.
+// Wavefronts with a stencil that leaves the mesh along x (clamped indices) move
+// those lanes' runs inside and their x weights along.
+// a stencil row: 3 ns words side by side, read 16 bytes at a time from any word
+template <typename T, int NS> struct M2PRow {
+  static constexpr int NW = 3 * NS * (int)sizeof(T) / 4, N4 = NW / 4, N1 = NW % 4;
+  typedef unsigned Quad __attribute__((ext_vector_type(4), aligned(4)));
+  typedef unsigned Pair __attribute__((ext_vector_type(2), aligned(4)));
+  static_assert(N1 == 0 || N1 == 2);
+  Quad q[N4];
+  Pair p;
+  __device__ __forceinline__ void load(const T *m) {
+    const unsigned *u = reinterpret_cast<const unsigned *>(m);
+#pragma unroll
+    for (int i = 0; i < N4; ++i) q[i] = *reinterpret_cast<const Quad *>(u + 4 * i);
+    if constexpr (N1 == 2) p = *reinterpret_cast<const Pair *>(u + 4 * N4);
+  }
+  __device__ __forceinline__ void get(T (&v)[NS][3]) const {
+    auto word = [&](int i) { return i < 4 * N4 ? q[i / 4][i % 4] : p[i % 2]; };
+#pragma unroll
+    for (int i = 0; i < 3 * NS; ++i) {
+      if constexpr (sizeof(T) == 8)
+        v[i / 3][i % 3] = __builtin_bit_cast(double, ((uint64_t)word(2 * i + 1) << 32) | word(2 * i));
+      else
+        v[i / 3][i % 3] = __builtin_bit_cast(float, word(i));
+    }
+  }
+};
+
 template <typename T, int NS>
 __global__ void __launch_bounds__(256) k_m2p(PGeom g, const T *mesh, const double *pos, NCount npc, double *out) {
   const int64_t np = npc.get();
   constexpr bool F64 = sizeof(T) == sizeof(double);
   constexpr bool M6 = NS == 6;
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
-    int idx[3][NS];
+    int idx[3][NS], i0x = 0;
     T w[3][NS];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -754,6 +791,7 @@ __global__ void __launch_bounds__(256) k_m2p(PGeom g, const T *mesh, const doubl
           w[d][s2] = weight_f(M6, s2, (float)dd);
         idx[d][s2] = b - g.off + s2;
       }
+      if (d == 0) i0x = b - g.off;
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -778,62 +816,127 @@ __global__ void __launch_bounds__(256) k_m2p(PGeom g, const T *mesh, const doubl
 #pragma unroll
     for (int s2 = 0; s2 < NS; ++s2) idx[1][s2] = min(max(idx[1][s2], g.lo[1]), g.hi[1]);
     double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    // node (sx, sy, sz) at row base (sy, sz) + x offset sx: one 64-bit base
-    // per stencil row, 32-bit offsets along x
-    int xo[NS];
+    // x run of the stencil: nodes xb .. xb + ns - 1 of the mesh, node j of it the
+    // stencil's j - k0 (k0 = 0: no x index clamped)
+    const int xb = min(max(i0x, g.lo[0]), g.hi[0] - NS + 1), k0 = i0x - xb;
+    // one stencil row's sums
+    auto add_row = [&](int r, const T (&mv)[NS][3]) {
+      const int sy = r % NS, sz = r / NS;
+      // FP32 form: the FP32 weights' product in FP64, y and z once per row
+      const double wyz = F64 ? 0.0 : (double)w[1][sy] * (double)w[2][sz];
 #pragma unroll
-    for (int sx = 0; sx < NS; ++sx) xo[sx] = 3 * (idx[0][sx] - g.lo[0]);
-    // stencil rows r = (sz, sy) in order, G rows at a time: a group's node
-    // triples are all loaded before any is summed (G ns gathers in flight per
-    // wavefront rather than one), and the scheduling barriers keep the
-    // compiler from moving loads back beside their uses or hoisting the next
-    // group's loads over this group's sums (register use stays bounded)
-    constexpr int G = F64 ? (M6 ? 1 : 2) : (M6 ? 2 : 4);
-#pragma unroll
-    for (int r0 = 0; r0 < NS * NS; r0 += G) {
-      T mv[G][NS][3];
-#pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const int sy = (r0 + k) % NS, sz = (r0 + k) / NS;
-        const int64_t row = (int64_t)g.E[0] * ((idx[1][sy] - g.lo[1]) + (int64_t)g.E[1] * (idx[2][sz] - g.lo[2]));
-        const T *mrow = mesh + 3 * row;
-#pragma unroll
-        for (int sx = 0; sx < NS; ++sx)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) mv[k][sx][c] = mrow[xo[sx] + c];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const int sy = (r0 + k) % NS, sz = (r0 + k) / NS;
-        // FP32 form: the FP32 weights' product in FP64, y and z once per row
-        const double wyz = F64 ? 0.0 : (double)w[1][sy] * (double)w[2][sz];
-#pragma unroll
-        for (int sx = 0; sx < NS; ++sx) {
-          const T *m = mv[k][sx];
-          if constexpr (F64) {
-            const double wt = __dmul_rn(__dmul_rn(w[0][sx], w[1][sy]), w[2][sz]);
-            const double t0 = __dmul_rn(wt, m[0]), t1 = __dmul_rn(wt, m[1]), t2 = __dmul_rn(wt, m[2]);
-            if (sz == 0 && sy == 0 && sx == 0) {   // the first term starts the sums
-              a0 = t0;
-              a1 = t1;
-              a2 = t2;
-            } else {
-              a0 = __dadd_rn(a0, t0);
-              a1 = __dadd_rn(a1, t1);
-              a2 = __dadd_rn(a2, t2);
-            }
+      for (int sx = 0; sx < NS; ++sx) {
+        const T *m = mv[sx];
+        if constexpr (F64) {
+          const double wt = __dmul_rn(__dmul_rn(w[0][sx], w[1][sy]), w[2][sz]);
+          const double t0 = __dmul_rn(wt, m[0]), t1 = __dmul_rn(wt, m[1]), t2 = __dmul_rn(wt, m[2]);
+          if (r == 0 && sx == 0) {   // the first term starts the sums
+            a0 = t0;
+            a1 = t1;
+            a2 = t2;
           } else {
-            // weight times FP32 node value fused into the FP64 sum
-            const double wt = (double)w[0][sx] * wyz;
-            a0 = __fma_rn(wt, (double)m[0], a0);
-            a1 = __fma_rn(wt, (double)m[1], a1);
-            a2 = __fma_rn(wt, (double)m[2], a2);
+            a0 = __dadd_rn(a0, t0);
+            a1 = __dadd_rn(a1, t1);
+            a2 = __dadd_rn(a2, t2);
           }
+        } else {
+          // weight times FP32 node value fused into the FP64 sum
+          const double wt = (double)w[0][sx] * wyz;
+          a0 = __fma_rn(wt, (double)m[0], a0);
+          a1 = __fma_rn(wt, (double)m[1], a1);
+          a2 = __fma_rn(wt, (double)m[2], a2);
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    // (indices and weights are hidden from the compiler in each of the two
+    // forms: it would form the rows' addresses and products ahead of both)
+    auto hide = [&] {
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+        asm volatile("" : "+v"(idx[1][t]), "+v"(idx[2][t]), "+v"(w[1][t]), "+v"(w[2][t]));
+    };
+    auto row_at = [&](int r) {
+      return 3 * ((int64_t)g.E[0] * ((idx[1][r % NS] - g.lo[1]) + (int64_t)g.E[1] * (idx[2][r / NS] - g.lo[2])));
+    };
+    // stencil rows r = (sz, sy) in order, G rows at a time: a group's rows are
+    // all loaded before any is summed, and the scheduling barriers keep the
+    // compiler from moving loads back beside their uses or hoisting the next
+    // group's loads over this group's sums (register use stays bounded)
+    constexpr int G = F64 ? (M6 ? 1 : 2) : 2;
+    auto sum_rows = [&](auto clamped) {
+      hide();
+      constexpr bool CL = decltype(clamped)::value;
+      const T *mx = mesh + 3 * (xb - g.lo[0]);
+      bool in[NS];   // node j of the run is one of the stencil's
+      if constexpr (CL) {
+        T wx[NS];
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+          in[j] = j - k0 >= 0 && j - k0 < NS;
+          wx[j] = (T)0;
+#pragma unroll
+          for (int t = 0; t < NS; ++t) wx[j] = j - k0 == t ? w[0][t] : wx[j];
+        }
+#pragma unroll
+        for (int j = 0; j < NS; ++j) w[0][j] = wx[j];
+      }
+#pragma unroll
+      for (int r0 = 0; r0 < NS * NS; r0 += G) {
+        M2PRow<T, NS> mv[G];
+#pragma unroll
+        for (int k = 0; k < G; ++k) mv[k].load(mx + row_at(r0 + k));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+          T v[NS][3];
+          mv[k].get(v);
+          if constexpr (CL) {
+            // the clamped nodes repeat the run's end with weight 0 (which an
+            // infinity or NaN there turns into NaN); a node of the run that is
+            // none of the stencil's adds nothing, whatever it holds
+            T e[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) e[c] = k0 == 0 ? (T)0 : (k0 < 0 ? v[0][c] : v[NS - 1][c]);
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+#pragma unroll
+              for (int c = 0; c < 3; ++c) v[j][c] = in[j] ? v[j][c] : (T)0;
+            add_row(r0 + k, v);
+            a0 += 0.0 * (double)e[0];
+            a1 += 0.0 * (double)e[1];
+            a2 += 0.0 * (double)e[2];
+          } else {
+            add_row(r0 + k, v);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto gather_rows = [&] {
+      hide();
+#pragma unroll
+      for (int r0 = 0; r0 < NS * NS; r0 += G) {
+        T mv[G][NS][3];
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+          const T *mrow = mesh + row_at(r0 + k);
+#pragma unroll
+          for (int sx = 0; sx < NS; ++sx)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) mv[k][sx][c] = mrow[3 * (idx[0][sx] - g.lo[0]) + c];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < G; ++k) add_row(r0 + k, mv[k]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (g.E[0] < NS)
+      gather_rows();
+    else if (__any(k0 != 0))
+      sum_rows(std::true_type());
+    else
+      sum_rows(std::false_type());
     out[3 * q] = a0;
     out[3 * q + 1] = a1;
     out[3 * q + 2] = a2;
