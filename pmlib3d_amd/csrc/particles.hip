@@ -34,10 +34,14 @@ struct Scratch {
 // Exclusive scan of n ints (in -> out, not aliased): out[0] = 0 and out[i +
 // 1] = in[0] + ... + in[i], so out[n] is the total.  Reduce, then scan, over
 // tiles of kIScanTile ints: the tile sums, one block turning them into tile
-// offsets, then each tile scanned through LDS (each thread a run of
-// kIScanItems) from its offset.  No memset, so a step may record it.
-constexpr int kIScanThreads = 256, kIScanItems = 16, kIScanTile = kIScanThreads * kIScanItems;
-constexpr int kIScanOffThreads = 1024;
+// offsets (up to kIScanFew tiles each tile adds the sums before it itself: one
+// launch less, 4 us of a recorded 64^3 step's scans of 11), then each tile
+// scanned through LDS (each thread a run of its share) from its offset.  No
+// memset, so a step may record it.  kIScanTile-int tiles, a quarter of that for
+// up to kIScanFew of these (300k ints: 73 tiles leave most CUs idle, 6 + 5 us
+// against 4 + 4).
+constexpr int kIScanThreads = 256, kIScanTile = 16 * kIScanThreads;
+constexpr int kIScanOffThreads = 1024, kIScanFew = 1024;
 __device__ __forceinline__ int block_excl_int(int v, int &total) {
   __shared__ int ws[kIScanThreads / 64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -59,11 +63,12 @@ __device__ __forceinline__ int block_excl_int(int v, int &total) {
   __syncthreads();   // ws is free for the next call
   return base + x - v;
 }
+template <int ITEMS>
 __global__ void __launch_bounds__(kIScanThreads) k_iscan_tiles(const int *in, int64_t n, int *tsum) {
-  const int64_t b = (int64_t)blockIdx.x * kIScanTile;
+  const int64_t b = (int64_t)blockIdx.x * (ITEMS * kIScanThreads);
   int s = 0;
 #pragma unroll
-  for (int j = 0; j < kIScanItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     const int64_t i = b + j * kIScanThreads + threadIdx.x;
     if (i < n) s += in[i];
   }
@@ -102,56 +107,76 @@ __global__ void __launch_bounds__(kIScanOffThreads) k_iscan_offsets(int *tsum, i
     run += __shfl(x, 63);
   }
 }
-__global__ void __launch_bounds__(kIScanThreads) k_iscan_apply(const int *in, int64_t n, const int *toff, int *out) {
-  __shared__ int sh[kIScanTile + kIScanTile / 32];
-  const int64_t b = (int64_t)blockIdx.x * kIScanTile;
+template <int ITEMS>
+__global__ void __launch_bounds__(kIScanThreads) k_iscan_apply(const int *in, int64_t n, const int *toff,
+                                                             int few, int *out) {
+  constexpr int TILE = ITEMS * kIScanThreads;
+  __shared__ int sh[TILE + TILE / 32];
+  const int64_t b = (int64_t)blockIdx.x * TILE;
   if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 #pragma unroll
-  for (int j = 0; j < kIScanItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     const int i = j * kIScanThreads + threadIdx.x;
     sh[i + i / 32] = b + i < n ? in[b + i] : 0;
   }
   __syncthreads();
-  int v[kIScanItems], sum = 0;
+  int v[ITEMS], sum = 0;
 #pragma unroll
-  for (int k = 0; k < kIScanItems; ++k) {
-    const int i = threadIdx.x * kIScanItems + k;
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = threadIdx.x * ITEMS + k;
     v[k] = sh[i + i / 32];
     sum += v[k];
   }
   int tot;
-  int run = block_excl_int(sum, tot) + toff[blockIdx.x];
+  int run = block_excl_int(sum, tot);
+  if (few) {   // toff holds the tiles' sums
+    int before = 0;
+    for (int t = threadIdx.x; t < (int)blockIdx.x; t += kIScanThreads) before += toff[t];
+    (void)block_excl_int(before, tot);
+    run += tot;
+  } else {
+    run += toff[blockIdx.x];
+  }
 #pragma unroll
-  for (int k = 0; k < kIScanItems; ++k) {
-    const int i = threadIdx.x * kIScanItems + k;
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = threadIdx.x * ITEMS + k;
     run += v[k];
     sh[i + i / 32] = run;
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kIScanItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     const int i = j * kIScanThreads + threadIdx.x;
     if (b + i < n) out[1 + b + i] = sh[i + i / 32];
   }
 }
-static int64_t iscan_tiles(int64_t n) { return (n + kIScanTile - 1) / kIScanTile; }
-// tsum: iscan_tiles(n) ints of scratch
+// ints of scratch of a scan of n (or fewer)
+static int64_t iscan_scratch(int64_t n) { return std::max<int64_t>((n + kIScanTile - 1) / kIScanTile, kIScanFew); }
+template <int ITEMS> static void iscan_run(const int *in, int *out, int64_t n, int64_t nt, int *tsum, hipStream_t st) {
+  const dim3 tiles((unsigned)nt);
+  const int few = nt <= kIScanFew;
+  hipLaunchKernelGGL(k_iscan_tiles<ITEMS>, tiles, dim3(kIScanThreads), 0, st, in, n, tsum);
+  if (!few) hipLaunchKernelGGL(k_iscan_offsets, dim3(1), dim3(kIScanOffThreads), 0, st, tsum, (int)nt);
+  hipLaunchKernelGGL(k_iscan_apply<ITEMS>, tiles, dim3(kIScanThreads), 0, st, in, n, (const int *)tsum, few, out);
+}
+// tsum: iscan_scratch(n) ints
 static int iscan_launch(const int *in, int *out, int64_t n, int *tsum, hipStream_t st) {
-  const int64_t nt = iscan_tiles(n);
+  const int64_t nt = (n + kIScanTile - 1) / kIScanTile, small = 4 * kIScanThreads;
   PM_CHECK(nt < (int64_t)1 << 31, "pmgpu: scan too large");
   if (nt == 0) {
     PM_HIP(hipMemsetAsync(out, 0, sizeof(int), st));
     return 0;
   }
-  hipLaunchKernelGGL(k_iscan_tiles, dim3((unsigned)nt), dim3(kIScanThreads), 0, st, in, n, tsum);
-  hipLaunchKernelGGL(k_iscan_offsets, dim3(1), dim3(kIScanOffThreads), 0, st, tsum, (int)nt);
-  hipLaunchKernelGGL(k_iscan_apply, dim3((unsigned)nt), dim3(kIScanThreads), 0, st, in, n, (const int *)tsum, out);
+  if (n <= small * kIScanFew)
+    iscan_run<4>(in, out, n, (n + small - 1) / small, tsum, st);
+  else
+    iscan_run<16>(in, out, n, nt, tsum, st);
   PM_HIP(hipGetLastError());
   return 0;
 }
 static int scan_exclusive(const int *in, int *out, int64_t n, Scratch &tmp, hipStream_t st) {
   PM_CHECK(in != out, "pmgpu: internal scan aliasing");
-  if (tmp.ensure(sizeof(int) * ((size_t)iscan_tiles(n) + 1))) return -1;
+  if (tmp.ensure(sizeof(int) * (size_t)iscan_scratch(n))) return -1;
   return iscan_launch(in, out, n, tmp.as<int>(), st);
 }
 
@@ -373,7 +398,7 @@ int p2m_device(const pmgpu_geom *geom, int prec, const double *xpart, const doub
   if (scan_exclusive(w.count.as<int>(), w.start.as<int>(), nbins, w.scan, st)) return -1;
   if (np > 0) {
     hipLaunchKernelGGL(k_p2m_scatter, grid_for(np), dim3(256), 0, st, np, nbins, key, rank, w.start.as<int>(),
-                       id_out);
+                       id_out, (int *)nullptr);
     PM_HIP(hipGetLastError());
   }
   const int accumulate = clear ? 0 : 1;
@@ -462,7 +487,8 @@ static void remesh_create_launch(const PGeom &g, int64_t nn, const int *flag, co
                                  const void *dvort_m, const void *vel_m, double *pos, double *vort, double *vel,
                                  double *dvort, double *vel_rk, double *dvort_rk, hipStream_t st) {
   hipLaunchKernelGGL(k_remesh_create<T>, grid_for(nn), dim3(256), 0, st, g, flag, offs, (const T *)vort_m,
-                     (const T *)dvort_m, (const T *)vel_m, pos, vort, vel, dvort, vel_rk, dvort_rk, INT64_MAX);
+                     (const T *)dvort_m, (const T *)vel_m, pos, vort, vel, dvort, vel_rk, dvort_rk, INT64_MAX,
+                     (int *)nullptr, (int *)nullptr);
 }
 
 int remesh_device(const pmgpu_geom *geom, int prec, const void *vort_m, const void *dvort_m, const void *vel_m,
@@ -960,53 +986,92 @@ struct Arr6 {
 };
 
 
-__global__ void k_fill_int(int *p, int64_t n, int v) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = v;
+// Three-way stable partition of the recorded step along an axis, gated: when
+// the stage's update left no particle outside the patch (or the axis moves
+// none), every kernel below returns at once.  The class of a particle is read
+// off its position wherever it is needed.  The class offsets come from a
+// two-level scan over tiles of kPartTile particles: the tiles' sums, then each
+// tile's own block scans in index order, from the sums before it (added by the
+// tile itself up to kPartFew tiles, beyond that by k_part_tile_scan).  A step
+// is bound by its launches, some 3 us each: three per axis (count, move, copy
+// back with the check) and one per stage for eight per axis and one per stage
+// (64^3 FP32, four steps: 1.93 -> 1.53 ms).
+constexpr int kPartFew = 1024;
+// counters of a stage, zero at its start
+struct StageState {
+  int outside;       // a particle left the patch
+  int counts[3][4];  // particles of each class along each axis
+};
+// the particles left when axis d's turn comes
+__device__ __forceinline__ int64_t stage_np(const int *np, const StageState *ss, int d) {
+  int n = *np;
+  for (int k = 0; k < d; ++k) n -= ss->counts[k][3];
+  return n;
 }
-// Three-way stable partition of the recorded step, gated: when the stage's
-// update left no particle outside the patch (or the axis moves none), every
-// kernel below returns at once.  The class offsets come from a two-level scan
-// over tiles of kPartTile particles (tile sums, one block scanning the tile
-// sums, then each tile's own block scans in index order), so that a step with
-// nothing to migrate launches no full-size scan.
-// class counts of each tile
-__global__ void __launch_bounds__(kPartThreads) k_part_tiles(NCount npc, const int *counts, const int *cls,
+// migration class along axis d: 0 stay, 1 west (wrap), 2 east (wrap), 3 drop
+struct PartAxis {
+  int d, per;
+  double lo, hi;
+  __device__ __forceinline__ int cls(const double *pos, int64_t q) const {
+    const double x = pos[3 * q + d];
+    const int c = x < lo ? 1 : (x >= hi ? 2 : 0);
+    return c != 0 && !per ? 3 : c;
+  }
+};
+// class counts of each tile and of all
+__global__ void __launch_bounds__(kPartThreads) k_part_count(const int *npp, StageState *ss, PartAxis ax, const double *pos,
                                                              Mig3 *tsum) {
-  if (part_idle(counts)) return;
-  const int64_t np = npc.get();
+  if (!ss->outside) return;
+  const int64_t np = stage_np(npp, ss, ax.d);
   Mig3 s{0, 0, 0};
 #pragma unroll
   for (int j = 0; j < kPartItems; ++j) {
     const int64_t q = (int64_t)blockIdx.x * kPartTile + j * kPartThreads + threadIdx.x;
-    if (q < np) s = m3_add(s, m3_of(cls[q]));
+    if (q < np) s = m3_add(s, m3_of(ax.cls(pos, q)));
   }
   Mig3 tot;
   (void)block_scan3(s, tot);
-  if (threadIdx.x == 0) tsum[blockIdx.x] = tot;
+  if (threadIdx.x == 0) {
+    tsum[blockIdx.x] = tot;
+    int *counts = ss->counts[ax.d];
+    if (tot.w) atomicAdd(&counts[1], tot.w);
+    if (tot.e) atomicAdd(&counts[2], tot.e);
+    if (tot.d) atomicAdd(&counts[3], tot.d);
+  }
 }
 // west movers, east movers, then stayers, each in their original order; a
-// stayer's rank is q minus the movers and drops before it
-__global__ void __launch_bounds__(kPartThreads) k_part_migrate(NCount npc, const int *cls, const Mig3 *toff,
-                                                               const int *counts, int d, double len, Arr6 src,
+// stayer's rank is q minus the movers and drops before it.  Moves what the
+// rest of the step reads: positions, strengths and the RK velocity.
+__global__ void __launch_bounds__(kPartThreads) k_part_migrate(const int *npp, const StageState *ss, PartAxis ax,
+                                                               const Mig3 *toff, int few, double len, Arr6 src,
                                                                Arr6 dst) {
+  const int *counts = ss->counts[ax.d];
   if (part_idle(counts)) return;
-  const int64_t np = npc.get();
+  const int64_t np = stage_np(npp, ss, ax.d);
   const int n1 = counts[1], n2 = counts[2];
-  Mig3 run = toff[blockIdx.x];
+  Mig3 run{0, 0, 0};
+  if (few) {   // toff holds the tiles' sums
+    for (int t = threadIdx.x; t < (int)blockIdx.x; t += kPartThreads) run = m3_add(run, toff[t]);
+    Mig3 tot;
+    (void)block_scan3(run, tot);
+    run = tot;
+  } else {
+    run = toff[blockIdx.x];
+  }
   for (int j = 0; j < kPartItems; ++j) {
     const int64_t q = (int64_t)blockIdx.x * kPartTile + j * kPartThreads + threadIdx.x;
-    const int c = q < np ? cls[q] : 0;
+    const int c = q < np ? ax.cls(src.a[0], q) : 0;
     Mig3 tot;
     const Mig3 ex = block_scan3(q < np ? m3_of(c) : Mig3{0, 0, 0}, tot);
     const Mig3 o = m3_add(run, ex);
     run = m3_add(run, tot);
     if (q >= np || c == 3) continue;
     const int64_t to = c == 1 ? o.w : (c == 2 ? n1 + o.e : n1 + n2 + (q - o.w - o.e - o.d));
-    for (int a = 0; a < 6; ++a) {
+#pragma unroll
+    for (int a = 0; a < 6; a += 2) {
       double v0 = src.a[a][3 * q], v1 = src.a[a][3 * q + 1], v2 = src.a[a][3 * q + 2];
       if (a == 0) {
-        double &x = d == 0 ? v0 : (d == 1 ? v1 : v2);
+        double &x = ax.d == 0 ? v0 : (ax.d == 1 ? v1 : v2);
         if (c == 1) x = x + len;
         if (c == 2) x = x - len;
       }
@@ -1016,29 +1081,26 @@ __global__ void __launch_bounds__(kPartThreads) k_part_migrate(NCount npc, const
     }
   }
 }
-__global__ void k_copy_back(NCount npc, const int *counts, Arr6 src, Arr6 dst) {
-  if (counts[1] + counts[2] + counts[3] == 0) return;
-  const int64_t n = 3 * (npc.get() - counts[3]);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    for (int a = 0; a < 6; ++a) dst.a[a][i] = src.a[a][i];
-}
-__global__ void k_np_drop(int *np, const int *counts) { *np -= counts[3]; }
-// a particle still outside a periodic axis after one wrap moved more than a
-// period in one stage: flagged (bit 2 of the status word)
-__global__ void k_check_inside(NCount npc, const int *outside, const double *pos, int d, double lo, double hi,
-                               int *err) {
-  if (!*outside) return;
-  const int64_t np = npc.get();
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
-    const double x = pos[3 * q + d];
-    if (x < lo || x >= hi) atomicOr(err, 2);
+// The moved set back into its arrays.  A particle still outside a periodic axis
+// after one wrap moved more than a period in one stage: flagged (bit 2 of the
+// status word).
+__global__ void k_copy_back(const int *npp, const StageState *ss, PartAxis ax, Arr6 src, Arr6 dst, int *err) {
+  const int *counts = ss->counts[ax.d];
+  if (part_idle(counts)) return;
+  const int64_t n = 3 * (stage_np(npp, ss, ax.d) - counts[3]);
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const double x = src.a[0][i];
+    if (ax.per && (x < ax.lo || x >= ax.hi) && i % 3 == ax.d) atomicOr(err, 2);
+    dst.a[0][i] = x;
+    dst.a[2][i] = src.a[2][i];
+    dst.a[4][i] = src.a[4][i];
   }
 }
-// the remeshed count, capped (bit 1 of the status word: over capacity)
-__global__ void k_np_from_offs(int *np, const int *offs, int64_t nn, int64_t cap, int *err) {
-  const int64_t t = offs[nn];
-  if (t > cap) atomicOr(err, 1);
-  *np = (int)(t > cap ? cap : t);
+// end of a stage (one thread): the dropped particles off the count, the
+// counters cleared for the next
+__global__ void k_stage_end(int *np, StageState *ss) {
+  *np = (int)stage_np(np, ss, 3);
+  *ss = StageState{};
 }
 
 struct VStep {
@@ -1066,7 +1128,6 @@ struct VStep {
   }
   int *d_np() { return state.as<int>(); }
   int *d_err() { return state.as<int>() + 1; }
-  int *d_outside() { return state.as<int>() + 2; }
   int ntiles() const { return (int)((cap + kPartTile - 1) / kPartTile); }
   void *mvort() { return mesh.p; }
   void *mvel() { return (char *)mesh.p + mesh_elems() * (prec == PMGPU_FP64 ? 8 : 4); }
@@ -1089,31 +1150,29 @@ struct VStep {
         w.rec.ensure(p2m_record_bytes(g, prec, cap)) || w.flag.ensure(sizeof(int) * (nn + 1)) ||
         w.offs.ensure(sizeof(int) * (nn + 1)))
       return -1;
-    const int64_t ts = iscan_tiles(nbins > nn ? nbins : nn);
-    if (w.scan.ensure(sizeof(int) * ((size_t)ts + 1))) return -1;
+    if (w.scan.ensure(sizeof(int) * (size_t)iscan_scratch(nbins > nn ? nbins : nn))) return -1;
     const size_t pb = sizeof(double) * 3 * (size_t)cap * 6;
     if (parts.ensure(pb) || tmp.ensure(pb) || mesh.ensure(2 * mesh_elems() * (prec == PMGPU_FP64 ? 8 : 4)) ||
-        mig.ensure(sizeof(int) * ((size_t)cap + 8) + sizeof(Mig3) * ((size_t)ntiles() + 1)) ||
+        mig.ensure(sizeof(StageState) + sizeof(Mig3) * ((size_t)ntiles() + 1)) ||
         state.ensure(sizeof(int) * 8))
       return -1;
     return 0;
   }
-  int *cls() { return mig.as<int>(); }
-  int *counts() { return mig.as<int>() + cap; }
-  Mig3 *toff() { return reinterpret_cast<Mig3 *>(mig.as<int>() + cap + 8); }
+  StageState *stage() { return mig.as<StageState>(); }
+  Mig3 *toff() { return reinterpret_cast<Mig3 *>(stage() + 1); }
 
-  // deposition of the particle vorticity onto the vorticity mesh (clear)
+  // deposition of the particle vorticity onto the vorticity mesh (clear); the
+  // bin counts are zero before and after
   int p2m() {
     const int nbins = g.nb[0] * g.nb[1] * g.nb[2];
     const NCount n(cap, d_np());
     Arr6 A = arrays(parts);
     int *key = w.key.as<int>(), *rank = w.ids.as<int>(), *id_out = rank + cap + 1;
-    hipLaunchKernelGGL(k_fill_int, grid_for(nbins + 1), dim3(256), 0, st, w.count.as<int>(), (int64_t)nbins + 1, 0);
     hipLaunchKernelGGL(k_p2m_keys, grid_for(cap), dim3(256), 0, st, g, (const double *)A.a[0], n, nbins, key, rank,
                        w.count.as<int>());
     if (iscan_launch(w.count.as<int>(), w.start.as<int>(), nbins, w.scan.as<int>(), st)) return -1;
-    hipLaunchKernelGGL(k_p2m_scatter, grid_for(cap), dim3(256), 0, st, n, nbins, key, rank, w.start.as<int>(),
-                       id_out);
+    hipLaunchKernelGGL(k_p2m_scatter, grid_for(std::max<int64_t>(cap, nbins)), dim3(256), 0, st, n, nbins, key, rank,
+                       w.start.as<int>(), id_out, w.count.as<int>());
     if (prec == PMGPU_FP64) {
       if (g.ns == 4) p2m_gather<double, 4>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
       else p2m_gather<double, 6>(g, A.a[0], A.a[2], cap, id_out, w, nbins, (double *)mvort(), 0, st);
@@ -1134,24 +1193,22 @@ struct VStep {
   }
 
   int migrate(int d) {
-    const NCount n(cap, d_np());
     Arr6 A = arrays(parts), T = arrays(tmp);
-    const double lo = geom.xmin[d], hi = geom.xmax[d], len = geom.xmax[d] - geom.xmin[d];
-    const int per = geom.bound_cond[d] != 0;
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, counts(), (int64_t)4, 0);
-    hipLaunchKernelGGL(k_classify, grid_for(cap), dim3(256), 0, st, n, (const int *)d_outside(),
-                       (const double *)A.a[0], d, lo, hi, per, cls(), counts());
+    const PartAxis ax{d, geom.bound_cond[d] != 0, geom.xmin[d], geom.xmax[d]};
     const dim3 tiles((unsigned)ntiles());
-    hipLaunchKernelGGL(k_part_tiles, tiles, dim3(kPartThreads), 0, st, n, (const int *)counts(), (const int *)cls(),
-                       toff());
-    hipLaunchKernelGGL(k_part_tile_scan, dim3(1), dim3(kTileScanThreads), 0, st, (const int *)counts(), toff(), ntiles());
-    hipLaunchKernelGGL(k_part_migrate, tiles, dim3(kPartThreads), 0, st, n, (const int *)cls(), (const Mig3 *)toff(),
-                       (const int *)counts(), d, len, A, T);
-    hipLaunchKernelGGL(k_copy_back, grid_for(3 * cap), dim3(256), 0, st, n, (const int *)counts(), T, A);
-    hipLaunchKernelGGL(k_np_drop, dim3(1), dim3(1), 0, st, d_np(), (const int *)counts());
-    if (per)
-      hipLaunchKernelGGL(k_check_inside, grid_for(cap), dim3(256), 0, st, NCount(cap, d_np()),
-                         (const int *)d_outside(), (const double *)A.a[0], d, lo, hi, d_err());
+    const int few = ntiles() <= kPartFew;
+    hipLaunchKernelGGL(k_part_count, tiles, dim3(kPartThreads), 0, st, (const int *)d_np(), stage(), ax,
+                       (const double *)A.a[0], toff());
+    if (!few)
+      hipLaunchKernelGGL(k_part_tile_scan, dim3(1), dim3(kTileScanThreads), 0, st, (const int *)stage()->counts[d],
+                         toff(), ntiles());
+    hipLaunchKernelGGL(k_part_migrate, tiles, dim3(kPartThreads), 0, st, (const int *)d_np(), (const StageState *)stage(), ax,
+                       (const Mig3 *)toff(), few, geom.xmax[d] - geom.xmin[d], A, T);
+    // (few blocks: mostly it has nothing to do, and an idle launch of 3000 takes twice one of 1000)
+    dim3 copy = grid_for(3 * cap);
+    copy.x = std::min(copy.x, 1024u);
+    hipLaunchKernelGGL(k_copy_back, copy, dim3(256), 0, st, (const int *)d_np(),
+                       (const StageState *)stage(), ax, T, A, d_err());
     PM_HIP(hipGetLastError());
     return 0;
   }
@@ -1184,13 +1241,14 @@ struct VStep {
         box.lo[d] = geom.xmin[d];
         box.hi[d] = geom.xmax[d];
       }
-      hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, d_outside(), (int64_t)1, 0);
       // no right-hand side in this step: dvort and dvort_rk stay zero
       hipLaunchKernelGGL(k_rk_update, grid_for(3 * cap), dim3(256), 0, st, k, dt, n, A.a[0], (const double *)A.a[1],
-                         A.a[2], (const double *)nullptr, A.a[4], (double *)nullptr, box, d_outside());
+                         A.a[2], (const double *)nullptr, A.a[4], (double *)nullptr, box, &stage()->outside);
       PM_HIP(hipGetLastError());
       for (int d = 0; d < 3; ++d)
         if (migrate(d)) return -1;
+      hipLaunchKernelGGL(k_stage_end, dim3(1), dim3(1), 0, st, d_np(), stage());
+      PM_HIP(hipGetLastError());
     }
     // remesh: deposit, flag, scan, create (velocity from the last stage's mesh)
     if (p2m()) return -1;
@@ -1203,13 +1261,11 @@ struct VStep {
     if (prec == PMGPU_FP64)
       hipLaunchKernelGGL(k_remesh_create<double>, grid_for(nn), dim3(256), 0, st, g, (const int *)w.flag.as<int>(),
                          (const int *)w.offs.as<int>(), (const double *)mvort(), (const double *)nullptr,
-                         (const double *)mvel(), A.a[0], A.a[2], A.a[1], A.a[3], A.a[4], A.a[5], cap);
+                         (const double *)mvel(), A.a[0], A.a[2], A.a[1], A.a[3], A.a[4], A.a[5], cap, d_np(), d_err());
     else
       hipLaunchKernelGGL(k_remesh_create<float>, grid_for(nn), dim3(256), 0, st, g, (const int *)w.flag.as<int>(),
                          (const int *)w.offs.as<int>(), (const float *)mvort(), (const float *)nullptr,
-                         (const float *)mvel(), A.a[0], A.a[2], A.a[1], A.a[3], A.a[4], A.a[5], cap);
-    hipLaunchKernelGGL(k_np_from_offs, dim3(1), dim3(1), 0, st, d_np(), (const int *)w.offs.as<int>(), nn, cap,
-                       d_err());
+                         (const float *)mvel(), A.a[0], A.a[2], A.a[1], A.a[3], A.a[4], A.a[5], cap, d_np(), d_err());
     PM_HIP(hipGetLastError());
     return 0;
   }
@@ -1273,6 +1329,8 @@ int pmgpu_vstep_create(const pmgpu_geom *g, const pmgpu_params *p, int32_t preci
   if (!e) e = s.prepare();
   if (!e && (hipMemsetAsync(s.state.p, 0, sizeof(int) * 8, s.st) != hipSuccess ||
              hipMemsetAsync(s.parts.p, 0, s.parts.cap, s.st) != hipSuccess ||
+             hipMemsetAsync(s.w.count.p, 0, s.w.count.cap, s.st) != hipSuccess ||
+             hipMemsetAsync(s.mig.p, 0, s.mig.cap, s.st) != hipSuccess ||
              hipStreamSynchronize(s.st) != hipSuccess)) {
     set_error("pmgpu_vstep_create: initialisation failed");
     e = -1;

@@ -165,12 +165,17 @@ static __global__ void k_p2m_keys(PGeom g, const double *pos, NCount npc, int nb
 }
 
 // counting-sort scatter: particle q to slot start[key] + rank of its bin
-static __global__ void k_p2m_scatter(NCount npc, int nbins, const int *key, const int *rank, const int *start, int *ids) {
+// clear (or null): the bin counts, set to zero for the next deposition
+static __global__ void k_p2m_scatter(NCount npc, int nbins, const int *key, const int *rank, const int *start, int *ids,
+                                     int *clear) {
   const int64_t np = npc.get();
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
     const int k = key[q];
     if (k < nbins) ids[start[k] + rank[q]] = (int)q;
   }
+  if (clear)
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k <= nbins; k += (int64_t)gridDim.x * blockDim.x)
+      clear[k] = 0;
 }
 
 // ascending order of ids[0, n) in place: insertion sort for the usual bins of
@@ -990,17 +995,23 @@ __global__ void k_remesh_flags(PGeom g, const T *vort, const T *dvort, const uin
 // A workgroup takes 256 consecutive cells at a time: their particles are one
 // contiguous range of the outputs, staged in LDS and then written with
 // consecutive threads on consecutive words.  Launched with 256 threads.
+// np (or null) takes the count, capped (err, bit 1: over capacity).
 constexpr int kRemeshTile = 256;
 template <typename T>
 __global__ void __launch_bounds__(kRemeshTile) k_remesh_create(PGeom g, const int *flag, const int *offs,
                                                                const T *vort, const T *dvort, const T *vel,
                                                                double *pos, double *pvort, double *pvel,
                                                                double *pdvort, double *vel_rk, double *dvort_rk,
-                                                               int64_t cap) {
+                                                               int64_t cap, int *np, int *err) {
   __shared__ double stage[4][3 * kRemeshTile];   // pos, vort, vel, dvort of the tile's particles
   const int64_t nn = (int64_t)g.E[0] * g.E[1] * g.E[2];
   const int64_t ntiles = (nn + kRemeshTile - 1) / kRemeshTile;
   const int tid = threadIdx.x;
+  if (np && blockIdx.x == 0 && tid == 0) {
+    const int64_t t = offs[nn];
+    if (t > cap) atomicOr(err, 1);
+    *np = (int)(t > cap ? cap : t);
+  }
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int64_t c0 = tile * kRemeshTile, idx = c0 + tid;
     const int64_t p0 = offs[c0], p1 = offs[min(c0 + kRemeshTile, nn)];
@@ -1077,21 +1088,6 @@ static __global__ void k_rk_update(RkCoef k, double dt, NCount npc, double *pos,
       const uint64_t m = __ballot(o);
       if (m && (threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1) atomicOr(outside, 1);
     }
-  }
-}
-
-// migration class along axis d: 0 stay, 1 west (wrap), 2 east (wrap), 3 drop;
-// nothing to do when the stage's update left every particle inside
-static __global__ void k_classify(NCount npc, const int *outside, const double *pos, int d, double lo, double hi,
-                                  int per, int *cls, int *counts) {
-  if (!*outside) return;
-  const int64_t np = npc.get();
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
-    double x = pos[3 * q + d];
-    int c = x < lo ? 1 : (x >= hi ? 2 : 0);
-    if (c != 0 && !per) c = 3;
-    cls[q] = c;
-    if (c != 0) atomicAdd(&counts[c], 1);
   }
 }
 
