@@ -31,14 +31,8 @@ template <typename T> struct PenArgs {
   T relax, cx, cy, cz;       // cx = 1 / (2 dx)
   T *vort;
   double *partial;           // 5 doubles per block, or null (no sums)
+  int zc;                    // planes per block
 };
-
-template <typename T>
-__device__ __forceinline__ T f_at(const PenArgs<T> &a, int64_t q, int c) {
-  T u = a.vel[3 * q + c];
-  T s = a.us ? a.us[3 * q + c] : (c == 0 ? a.us0 : (c == 1 ? a.us1 : a.us2));
-  return rmul(a.chi[q], rsub(s, u));
-}
 
 // central difference from the values at offsets -2, -1, +1, +2 (FD = 4) or
 // -1, +1 (FD = 2; m2 and p2 unused)
@@ -60,22 +54,33 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-constexpr int kTx = 64, kTy = 4;
-constexpr int kZc = 16;   // planes per workgroup
+constexpr int kTx = 64, kTy = 8;
+constexpr int kZc = 32;   // most planes per workgroup
 
 // A workgroup of kTx x kTy threads owns an (i, j) tile of interior cells and
-// walks the planes of its z chunk (kZc planes).  Per plane it forms f once
-// for the tile and an H = fd/2 halo in x and y into LDS; the x and y
-// differences come from there, the z differences from a per-thread queue of
-// the cell's f0 and f1 over the 2H + 1 planes around it, so a plane's
-// vorticity is finished H planes after it was formed.  Per cell the operations
-// and their order are those of the reference's loop, so the FP64 result is
-// bit-identical to it; the sums are formed per (i tile, j tile, plane) and
-// reduced in a fixed order.
+// walks the planes of its z chunk (zc planes).  Per plane it forms f once for
+// the tile and the H = fd/2 halo rows and columns the differences reach (not
+// the corners): a thread its own cell, and up to two thirds of them one halo
+// cell, the next plane's values loaded while this one's are differenced.  f
+// goes through LDS (two planes in turn, one barrier each) for the x and y
+// differences, the z differences come from a per-thread queue of the cell's f0
+// and f1 over the 2H + 1 planes around it, so a plane's vorticity is finished H
+// planes after it was formed.  Per cell the operations and their order are
+// those of the reference's loop, so the FP64 result is bit-identical to it; the
+// sums are formed per thread over its planes, then per workgroup in a fixed
+// order.
+// What bounds it: memory, 104 B per cell and the halos, of which the tile
+// re-reads (2H (kTx + kTy)) / (kTx kTy) from L2 and the chunk 2H / zc from
+// memory: 252^3 FP64 403 us, 1.66 GB of its own at 4.1 TB/s (64 x 4 tiles of 16
+// planes with whole halo rings, two barriers and a reduction of the sums per
+// plane: 555 us).
+template <typename T> struct PenCell {
+  T u[3], s[3], chi;
+};
 template <typename T, int FD>
 __global__ void __launch_bounds__(kTx *kTy) k_penalise(PenArgs<T> a) {
   constexpr int H = FD / 2, TW = kTx + 2 * H, TH = kTy + 2 * H, Q = 2 * H + 1;
-  __shared__ T fl[3][TH][TW];
+  __shared__ T fl_all[2][3][TH][TW];
   __shared__ double red[kTy][5];
   const BGeom &g = a.g;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * kTx + tx;
@@ -86,11 +91,36 @@ __global__ void __launch_bounds__(kTx *kTy) k_penalise(PenArgs<T> a) {
             bz = (int)(lt / ((int64_t)gridDim.x * gridDim.y));
   const int i0 = bx * kTx + 1, j0 = by * kTy + 1;   // interior indices are 1..N
   const int i = i0 + tx, j = j0 + ty;
-  const int k0 = bz * kZc + 1, k1 = min(k0 + kZc - 1, g.N[2]);
+  const int k0 = bz * a.zc + 1, k1 = min(k0 + a.zc - 1, g.N[2]);
   const bool own = i <= g.N[0] && j <= g.N[1];
   const int64_t sy = g.E[0], sz = (int64_t)g.E[0] * g.E[1];
   auto cell = [&](int ii, int jj, int kk) {
     return (int64_t)(ii - 1 + g.ng[0]) + sy * (jj - 1 + g.ng[1]) + sz * (kk - 1 + g.ng[2]);
+  };
+  // the thread's halo cell: rows below and above the tile, then columns beside
+  // it (cells no owned cell reaches are skipped: they may lie past the ghost
+  // layers)
+  int hr, hc;
+  if (tid < 2 * H * kTx) {
+    hr = tid / kTx;
+    hr = hr < H ? hr : hr + kTy;
+    hc = tid % kTx + H;
+  } else {
+    const int q = tid - 2 * H * kTx;
+    hr = q / (2 * H) + H;
+    hc = q % (2 * H);
+    hc = hc < H ? hc : hc + kTx;
+  }
+  static_assert(2 * H * (kTx + kTy) <= kTx * kTy);
+  const bool halo = tid < 2 * H * (kTx + kTy) && i0 - H + hc <= g.N[0] + H && j0 - H + hr <= g.N[1] + H;
+  const bool centre = i <= g.N[0] + H && j <= g.N[1] + H;
+  auto load = [&](PenCell<T> &p, int64_t q) {
+    p.chi = a.chi[q];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      p.u[m] = a.vel[3 * q + m];
+      p.s[m] = a.us ? a.us[3 * q + m] : (m == 0 ? a.us0 : (m == 1 ? a.us1 : a.us2));
+    }
   };
   T q0[Q], q1[Q];        // f0, f1 of the own cell, oldest plane first
   T pend[H + 1][4];      // dvdx, dwdx, dudy, dwdy of the planes not yet finished
@@ -100,17 +130,32 @@ __global__ void __launch_bounds__(kTx *kTy) k_penalise(PenArgs<T> a) {
   for (int t = 0; t <= H; ++t)
 #pragma unroll
     for (int c = 0; c < 4; ++c) pend[t][c] = T(0);
+  double s[5] = {0, 0, 0, 0, 0};
+  PenCell<T> pc{}, ph{};
+  const int64_t qc0 = centre ? cell(i, j, k0 - H) : 0, qh0 = halo ? cell(i0 - H + hc, j0 - H + hr, k0 - H) : 0;
+  if (centre) load(pc, qc0);
+  if (halo) load(ph, qh0);
   for (int kk = k0 - H; kk <= k1 + H; ++kk) {
-    // f of the tile and its halo at plane kk (cells no owned cell reaches are
-    // skipped: they may lie past the ghost layers)
-    for (int idx = tid; idx < TW * TH; idx += kTx * kTy) {
-      const int r = idx / TW, c = idx - r * TW;
-      const int ii = i0 - H + c, jj = j0 - H + r;
-      if (ii <= g.N[0] + H && jj <= g.N[1] + H) {
-        const int64_t q = cell(ii, jj, kk);
+    T(*fl)[TH][TW] = fl_all[(kk - k0 + H) & 1];
+    if (centre) {
 #pragma unroll
-        for (int m = 0; m < 3; ++m) fl[m][r][c] = f_at(a, q, m);
-      }
+      for (int m = 0; m < 3; ++m) fl[m][ty + H][tx + H] = rmul(pc.chi, rsub(pc.s[m], pc.u[m]));
+    }
+    if (halo) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) fl[m][hr][hc] = rmul(ph.chi, rsub(ph.s[m], ph.u[m]));
+    }
+    // the plane finished below, and the next plane's cells
+    const int kf = kk - H;
+    T *const v = a.vort + (own && kf >= k0 ? 3 * cell(i, j, kf) : 0);
+    T vo[3] = {T(0), T(0), T(0)};
+    if (own && kf >= k0) {
+#pragma unroll
+      for (int m = 0; m < 3; ++m) vo[m] = v[m];
+    }
+    if (kk < k1 + H) {
+      if (centre) load(pc, qc0 + sz * (kk + 1 - k0 + H));
+      if (halo) load(ph, qh0 + sz * (kk + 1 - k0 + H));
     }
     __syncthreads();
 #pragma unroll
@@ -118,10 +163,10 @@ __global__ void __launch_bounds__(kTx *kTy) k_penalise(PenArgs<T> a) {
       q0[t] = q0[t + 1];
       q1[t] = q1[t + 1];
     }
-    q0[Q - 1] = fl[0][ty + H][tx + H];
-    q1[Q - 1] = fl[1][ty + H][tx + H];
+    const int r = ty + H, c = tx + H;
+    q0[Q - 1] = fl[0][r][c];
+    q1[Q - 1] = fl[1][r][c];
     if (kk >= k0 && kk <= k1) {
-      const int r = ty + H, c = tx + H;
       const T x2 = H == 2 ? fl[1][r][c - 2] : T(0), x_2 = H == 2 ? fl[1][r][c + 2] : T(0);
       const T z2 = H == 2 ? fl[2][r][c - 2] : T(0), z_2 = H == 2 ? fl[2][r][c + 2] : T(0);
       pend[H][0] = cdiff_v<T, FD>(x2, fl[1][r][c - 1], fl[1][r][c + 1], x_2, a.cx);   // dv/dx
@@ -131,60 +176,52 @@ __global__ void __launch_bounds__(kTx *kTy) k_penalise(PenArgs<T> a) {
       pend[H][2] = cdiff_v<T, FD>(y2, fl[0][r - 1][c], fl[0][r + 1][c], y_2, a.cy);   // du/dy
       pend[H][3] = cdiff_v<T, FD>(w2, fl[2][r - 1][c], fl[2][r + 1][c], w_2, a.cy);   // dw/dy
     }
-    __syncthreads();   // the tile is read; the next plane may overwrite it
-    const int kf = kk - H;   // plane finished now
-    if (kf >= k0) {
-      double s[5] = {0, 0, 0, 0, 0};
-      if (own) {
-        const T dvdx = pend[0][0], dwdx = pend[0][1], dudy = pend[0][2], dwdy = pend[0][3];
-        const T dudz = cdiff_v<T, FD>(q0[0], q0[H - 1], q0[H + 1], q0[Q - 1], a.cz);
-        const T dvdz = cdiff_v<T, FD>(q1[0], q1[H - 1], q1[H + 1], q1[Q - 1], a.cz);
-        T w0 = rmul(a.relax, rsub(dwdy, dvdz));
-        T w1 = rmul(a.relax, rsub(dudz, dwdx));
-        T w2 = rmul(a.relax, rsub(dvdx, dudy));
-        T *v = a.vort + 3 * cell(i, j, kf);
-        T v0 = radd(v[0], w0), v1 = radd(v[1], w1), v2 = radd(v[2], w2);
-        v[0] = v0;
-        v[1] = v1;
-        v[2] = v2;
-        if (a.partial) {
-          const double px = __dadd_rn(g.xmin[0], __dmul_rn(__dadd_rn((double)(i - 1), 0.5), g.dx[0]));
-          const double py = __dadd_rn(g.xmin[1], __dmul_rn(__dadd_rn((double)(j - 1), 0.5), g.dx[1]));
-          const double pz = __dadd_rn(g.xmin[2], __dmul_rn(__dadd_rn((double)(kf - 1), 0.5), g.dx[2]));
-          const double d0 = w0, d1 = w1, d2 = w2, e0 = v0, e1 = v1, e2 = v2;
-          s[0] = __dsub_rn(__dmul_rn(py, d2), __dmul_rn(pz, d1));
-          s[1] = __dsub_rn(__dmul_rn(pz, d0), __dmul_rn(px, d2));
-          s[2] = __dsub_rn(__dmul_rn(px, d1), __dmul_rn(py, d0));
-          s[3] = __dadd_rn(__dadd_rn(__dmul_rn(d0, d0), __dmul_rn(d1, d1)), __dmul_rn(d2, d2));
-          s[4] = __dadd_rn(__dadd_rn(__dmul_rn(e0, e0), __dmul_rn(e1, e1)), __dmul_rn(e2, e2));
-        }
-      }
+    if (own && kf >= k0) {
+      const T dvdx = pend[0][0], dwdx = pend[0][1], dudy = pend[0][2], dwdy = pend[0][3];
+      const T dudz = cdiff_v<T, FD>(q0[0], q0[H - 1], q0[H + 1], q0[Q - 1], a.cz);
+      const T dvdz = cdiff_v<T, FD>(q1[0], q1[H - 1], q1[H + 1], q1[Q - 1], a.cz);
+      T w0 = rmul(a.relax, rsub(dwdy, dvdz));
+      T w1 = rmul(a.relax, rsub(dudz, dwdx));
+      T w2 = rmul(a.relax, rsub(dvdx, dudy));
+      T v0 = radd(vo[0], w0), v1 = radd(vo[1], w1), v2 = radd(vo[2], w2);
+      v[0] = v0;
+      v[1] = v1;
+      v[2] = v2;
       if (a.partial) {
-        for (int m = 0; m < 5; ++m) {
-          double t = wave_sum(s[m]);
-          if (tx == 0) red[ty][m] = t;
-        }
-        __syncthreads();
-        if (ty == 0 && tx < 5) {
-          double t = 0.0;
-          for (int w = 0; w < kTy; ++w) t += red[w][tx];
-          // the block index of the (i tile, j tile, plane) partial
-          const int64_t b = bx + (int64_t)gridDim.x * (by + (int64_t)gridDim.y * (kf - 1));
-          a.partial[5 * b + tx] = t;
-        }
-        __syncthreads();
+        const double px = __dadd_rn(g.xmin[0], __dmul_rn(__dadd_rn((double)(i - 1), 0.5), g.dx[0]));
+        const double py = __dadd_rn(g.xmin[1], __dmul_rn(__dadd_rn((double)(j - 1), 0.5), g.dx[1]));
+        const double pz = __dadd_rn(g.xmin[2], __dmul_rn(__dadd_rn((double)(kf - 1), 0.5), g.dx[2]));
+        const double d0 = w0, d1 = w1, d2 = w2, e0 = v0, e1 = v1, e2 = v2;
+        s[0] += __dsub_rn(__dmul_rn(py, d2), __dmul_rn(pz, d1));
+        s[1] += __dsub_rn(__dmul_rn(pz, d0), __dmul_rn(px, d2));
+        s[2] += __dsub_rn(__dmul_rn(px, d1), __dmul_rn(py, d0));
+        s[3] += __dadd_rn(__dadd_rn(__dmul_rn(d0, d0), __dmul_rn(d1, d1)), __dmul_rn(d2, d2));
+        s[4] += __dadd_rn(__dadd_rn(__dmul_rn(e0, e0), __dmul_rn(e1, e1)), __dmul_rn(e2, e2));
       }
     }
 #pragma unroll
     for (int t = 0; t < H; ++t)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) pend[t][c] = pend[t + 1][c];
+      for (int c2 = 0; c2 < 4; ++c2) pend[t][c2] = pend[t + 1][c2];
+  }
+  if (a.partial) {
+    for (int m = 0; m < 5; ++m) {
+      double t = wave_sum(s[m]);
+      if (tx == 0) red[ty][m] = t;
+    }
+    __syncthreads();
+    if (ty == 0 && tx < 5) {
+      double t = 0.0;
+      for (int w = 0; w < kTy; ++w) t += red[w][tx];
+      a.partial[5 * (bx + (int64_t)gridDim.x * (by + (int64_t)gridDim.y * bz)) + tx] = t;
+    }
   }
 }
 
 // fixed-order reduction of the per-block sums (one block): thread t adds the
 // blocks t, t + 256, ... in that order, then a fixed tree; the loads of 8
-// blocks are issued ahead of their adds
+// blocks are issued ahead of their adds (252^3: 1024 blocks, 6 us;
+// with a sum per 64 x 4 cells of a plane 71 us)
 __global__ void __launch_bounds__(256) k_penalise_sums(const double *partial, int64_t nb, double *out) {
   __shared__ double sh[5][256];
   double t[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -216,14 +253,18 @@ __global__ void __launch_bounds__(256) k_penalise_sums(const double *partial, in
 
 constexpr int kMaxDevices = 64;
 
-// workgroups of k_penalise; the partial sums are one per (i tile, j tile,
-// plane), partial_blocks of them
-static dim3 penalise_grid(const pmgpu_geom *geom) {
-  return dim3((geom->ncell[0] + kTx - 1) / kTx, (geom->ncell[1] + kTy - 1) / kTy, (geom->ncell[2] + kZc - 1) / kZc);
+// workgroups of k_penalise: chunks of kZc planes, fewer on a mesh that leaves
+// CUs idle (two workgroups per CU; each chunk re-reads fd planes)
+static dim3 penalise_grid(const pmgpu_geom *geom, int &zc) {
+  const int64_t tiles = (int64_t)((geom->ncell[0] + kTx - 1) / kTx) * ((geom->ncell[1] + kTy - 1) / kTy);
+  zc = kZc;
+  while (zc > 4 && tiles * ((geom->ncell[2] + zc - 1) / zc) < 512) zc /= 2;
+  return dim3((geom->ncell[0] + kTx - 1) / kTx, (geom->ncell[1] + kTy - 1) / kTy, (geom->ncell[2] + zc - 1) / zc);
 }
+// partial sums a call may need (one per workgroup) and the limit of the calls
+// with a fixed buffer: one per 64 x 4 cells of a plane
 static int64_t partial_blocks(const pmgpu_geom *geom) {
-  const dim3 g = penalise_grid(geom);
-  return (int64_t)g.x * g.y * geom->ncell[2];
+  return (int64_t)((geom->ncell[0] + 63) / 64) * ((geom->ncell[1] + 3) / 4) * geom->ncell[2];
 }
 
 struct PenWS {
@@ -276,9 +317,9 @@ static int penalise_run(const pmgpu_geom *geom, const void *vel, const void *chi
   a.cz = T(1.0) / (T(2.0) * T(geom->dx[2]));
   a.vort = (T *)vort;
   PM_CHECK(geom->ncell[2] < 65536 && geom->ncell[1] < (1 << 20), "pmgpu_penalise: mesh too large");
-  const dim3 grid = penalise_grid(geom);
-  const int64_t nb = partial_blocks(geom);
-  PM_CHECK(!partial || nb <= cap, "pmgpu_penalise: more blocks than the partial-sum buffer holds");
+  const dim3 grid = penalise_grid(geom, a.zc);
+  const int64_t nb = (int64_t)grid.x * grid.y * grid.z;
+  PM_CHECK(!partial || partial_blocks(geom) <= cap, "pmgpu_penalise: more blocks than the partial-sum buffer holds");
   a.partial = partial;
   if (fd_order == 4)
     hipLaunchKernelGGL((k_penalise<T, 4>), grid, dim3(kTx, kTy), 0, st, a);
