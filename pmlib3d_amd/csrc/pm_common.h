@@ -26,6 +26,10 @@ template <typename V> __device__ __forceinline__ V cmul(V a, V b) {
 }
 template <typename V> __device__ __forceinline__ V cconj(V a) { return cmake<V>(a.x, -a.y); }
 template <typename V, typename R> __device__ __forceinline__ V cscale(V a, R s) { return cmake<V>(a.x * s, a.y * s); }
+// a s + c (fused where the file is compiled with contraction)
+template <typename V, typename R> __device__ __forceinline__ V cmadd(V a, R s, V c) {
+  return cmake<V>(a.x * s + c.x, a.y * s + c.y);
+}
 // multiply by i*s with s = +1 or -1 (compile time)
 template <int S, typename V> __device__ __forceinline__ V cmul_i(V a) {
   return S > 0 ? cmake<V>(-a.y, a.x) : cmake<V>(a.y, -a.x);

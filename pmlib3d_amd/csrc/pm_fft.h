@@ -57,17 +57,18 @@ template <int S, typename V> struct Dft<8, S, V> {
       a[k] = cadd(v[k], v[k + 4]);
       b[k] = csub(v[k], v[k + 4]);
     }
-    // b[k] *= exp(S * 2 pi i k / 8)
-    b[1] = cscale(cadd(b[1], cmul_i<S>(b[1])), h);
-    b[2] = cmul_i<S>(b[2]);
-    b[3] = cscale(csub(cmul_i<S>(b[3]), b[3]), h);
+    // b[k] *= exp(S * 2 pi i k / 8), the radix-4 transform of the products with
+    // the 1 / sqrt 2 of b[1] and b[3] left to its last sums
+    const V p1 = cadd(b[1], cmul_i<S>(b[1])), p3 = csub(cmul_i<S>(b[3]), b[3]);
+    const V p2 = cmul_i<S>(b[2]);
+    const V s02 = cadd(b[0], p2), d02 = csub(b[0], p2), s13 = cadd(p1, p3), d13 = cmul_i<S>(csub(p1, p3));
     Dft<4, S, V>::run(a);
-    Dft<4, S, V>::run(b);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      v[2 * m] = a[m];
-      v[2 * m + 1] = b[m];
-    }
+    for (int m = 0; m < 4; ++m) v[2 * m] = a[m];
+    v[1] = cmadd(s13, h, s02);
+    v[3] = cmadd(d13, h, d02);
+    v[5] = cmadd(s13, -h, s02);
+    v[7] = cmadd(d13, -h, d02);
   }
 };
 
