@@ -1081,7 +1081,10 @@ static __global__ void k_rk_update(RkCoef k, double dt, NCount npc, double *pos,
       dvort_rk[i] = dr;
       vort[i] = __dadd_rn(vort[i], __dmul_rn(k.c2, dr));
     } else {
-      vort[i] = __dadd_rn(vort[i], dinc);
+      // (a zero increment changes -0 only: the store, 8 of 56 bytes per word,
+      // falls away otherwise; 384^3 1.90 -> 1.56 ms)
+      const double v = vort[i], w = __dadd_rn(v, dinc);
+      if (__double_as_longlong(w) != __double_as_longlong(v)) vort[i] = w;
     }
     if (outside) {
       const bool o = x < box.lo[d] || x >= box.hi[d];
