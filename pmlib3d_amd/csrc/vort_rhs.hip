@@ -21,17 +21,27 @@ template <typename T> struct RhsArgs {
   T *dw;
   int E[3], N[3], ng[3];
   T visc, cdx2[3], c2dx[3];  // 1 / dx^2 and 1 / (2 dx) per axis
+  int planes;                // per workgroup
 };
 
 // One thread per component word of kRows rows (consecutive threads own
 // consecutive words of a row, components fastest); a block covers kRowWords
-// words of kRows consecutive rows and marches through kPlanes planes.  Each
+// words of kRows consecutive rows and marches through some planes.  Each
 // thread keeps its words' values on the planes within H = FD / 2 of the
 // current one in registers (one new plane loaded per step); the current
-// plane's tile with an H-cell halo in x and y is staged in LDS (the centre
-// from those registers, the halo from memory), and the x and y stencils read
-// it there.
-constexpr int kRowWords = 256, kRows = 4, kPlanes = 16;
+// plane's tile with its halo in x and y (H rows above and below, 3 H words
+// beside the rows, no corners) is staged in LDS, the centre from those
+// registers, the halo from memory (four words of rows a thread and one of the
+// sides, at offsets kept from plane to plane), and the x and y stencils read it
+// there.  The loads of the next plane are in flight while this one is summed.
+// What bounds it: memory, and the rows that neighbouring tiles read again
+// (2 H / kRows of them, from L2): 160^3 FP32 61 us for 147 MB of its own, FP64
+// 101 us (with the halo's words found and loaded anew behind each plane's
+// barrier 83 and 183 us).
+constexpr int kRowWords = 256, kRows = 4;
+// planes per workgroup, halved down to 2 while the chip has not two workgroups
+// per CU (64^3 FP32 28 us with 16, 8 us with 2)
+constexpr int kPlanes = 16;
 
 template <typename T, int FD>
 __global__ void __launch_bounds__(kRowWords) k_vort_rhs(RhsArgs<T> a) {
@@ -47,7 +57,7 @@ __global__ void __launch_bounds__(kRowWords) k_vort_rhs(RhsArgs<T> a) {
   const int x3 = x0 + tid, nw = 3 * a.N[0];      // this thread's word, words per row
   const bool mine = x3 < nw;
   const int l = x3 % 3;
-  const int k0 = kz * kPlanes, k1 = k0 + kPlanes < a.N[2] ? k0 + kPlanes : a.N[2];
+  const int k0 = kz * a.planes, k1 = k0 + a.planes < a.N[2] ? k0 + a.planes : a.N[2];
   const int64_t sy = 3 * (int64_t)a.E[0], sz = 3 * (int64_t)a.E[0] * a.E[1];
   // word wd (interior-relative, may be a halo word), row jj, plane kk
   auto at = [&](int wd, int jj, int kk) {
@@ -64,6 +74,45 @@ __global__ void __launch_bounds__(kRowWords) k_vort_rhs(RhsArgs<T> a) {
       zw[r][m + 1] = ok ? a.w[at(x3, j0 + r, k0 + m - H)] : T(0);
       zu[r][m + 1] = ok ? a.u[at(x3, j0 + r, k0 + m - H)] : T(0);
     }
+  // the thread's halo words: place in the tile, offset from plane 0 of the mesh
+  constexpr int NH = 2 * H + 1;
+  int hl[NH];
+  int64_t hg[NH];
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    int rr, c;
+    bool ok = true;
+    if (i + 1 < NH) {
+      rr = i < H ? i : i + kRows;
+      c = HW + tid;
+    } else {
+      rr = H + tid / (2 * HW);
+      c = tid % (2 * HW);
+      c = c < HW ? c : c + kRowWords;
+      ok = tid < kRows * 2 * HW;
+    }
+    const int wd = x0 - HW + c, jj = j0 - H + rr;
+    ok = ok && wd < nw + HW && jj < a.N[1] + H;
+    hl[i] = ok ? rr * TW + c : -1;
+    hg[i] = ok ? at(wd, jj, 0) : 0;
+  }
+  T hw[NH], hu[NH], nw_[kRows], nu_[kRows];   // the next plane's halo, and the queues' next values
+  int64_t cg[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) cg[r] = x3 < nw + HW && j0 + r < a.N[1] + H ? at(x3, j0 + r, 0) : -1;
+  auto load = [&](int k) {
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+      hw[i] = hl[i] >= 0 ? a.w[hg[i] + sz * k] : T(0);
+      hu[i] = hl[i] >= 0 ? a.u[hg[i] + sz * k] : T(0);
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      nw_[r] = cg[r] >= 0 ? a.w[cg[r] + sz * (k + H)] : T(0);
+      nu_[r] = cg[r] >= 0 ? a.u[cg[r] + sz * (k + H)] : T(0);
+    }
+  };
+  load(k0);
   for (int k = k0; k < k1; ++k) {
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
@@ -72,23 +121,18 @@ __global__ void __launch_bounds__(kRowWords) k_vort_rhs(RhsArgs<T> a) {
         zw[r][m] = zw[r][m + 1];
         zu[r][m] = zu[r][m + 1];
       }
-      const bool ok = x3 < nw + HW && j0 + r < a.N[1] + H;
-      zw[r][2 * H] = ok ? a.w[at(x3, j0 + r, k + H)] : T(0);
-      zu[r][2 * H] = ok ? a.u[at(x3, j0 + r, k + H)] : T(0);
+      zw[r][2 * H] = nw_[r];
+      zu[r][2 * H] = nu_[r];
       lw[H + r][HW + tid] = zw[r][H];
       lu[H + r][HW + tid] = zu[r][H];
     }
-    // halo: H rows above and below (whole tile width), HW words left and
-    // right of the centre rows; positions outside the mesh are not needed
-    for (int idx = tid; idx < TR * TW; idx += kRowWords) {
-      const int rr = idx / TW, c = idx - rr * TW;
-      if (rr >= H && rr < H + kRows && c >= HW && c < HW + kRowWords) continue;  // centre
-      const int wd = x0 - HW + c, jj = j0 - H + rr;
-      if (wd >= -HW && wd < nw + HW && jj >= -H && jj < a.N[1] + H) {
-        lw[rr][c] = a.w[at(wd, jj, k)];
-        lu[rr][c] = a.u[at(wd, jj, k)];
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+      if (hl[i] >= 0) {
+        lw[0][hl[i]] = hw[i];
+        lu[0][hl[i]] = hu[i];
       }
-    }
+    if (k + 1 < k1) load(k + 1);
     __syncthreads();
     if (mine) {
 #pragma unroll
@@ -159,8 +203,11 @@ static int vort_rhs_launch(const pmgpu_geom *geom, const void *w, const void *u,
   a.visc = T(visc);
   if ((int64_t)a.N[0] * a.N[1] * a.N[2] > 0) {
     PM_CHECK(a.N[1] / kRows < 65535 && a.N[2] / kPlanes < 65535, "pmgpu_vorticity_rhs: mesh too large");
+    const int64_t tiles = (int64_t)((3 * a.N[0] + kRowWords - 1) / kRowWords) * ((a.N[1] + kRows - 1) / kRows);
+    a.planes = kPlanes;
+    while (a.planes > 2 && tiles * ((a.N[2] + a.planes - 1) / a.planes) < 512) a.planes /= 2;
     const dim3 grid((3 * a.N[0] + kRowWords - 1) / kRowWords, (a.N[1] + kRows - 1) / kRows,
-                    (a.N[2] + kPlanes - 1) / kPlanes);
+                    (a.N[2] + a.planes - 1) / a.planes);
     if (fd_order == 4)
       hipLaunchKernelGGL((k_vort_rhs<T, 4>), grid, dim3(kRowWords), 0, st, a);
     else
