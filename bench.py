@@ -633,7 +633,7 @@ def diagnostics_benchmark(reps, n=128):
     return res
 
 
-Z_KERNEL = "k_z3_r<float, 512, 4, false, true>"
+Z_KERNEL = "k_z3_r<float, 512, 4, false, true, 0>"
 
 
 def multires_benchmark(reps, n=256):

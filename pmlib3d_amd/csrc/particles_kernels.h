@@ -2,12 +2,13 @@
 // remeshing and the low-storage RK update with one-rank migration.
 //
 // Deposition is a gather, not a scatter: particles are binned by the cell of
-// their stencil base index (bit-exact NINT), a stable radix sort orders
-// them by bin and, inside a bin, by particle id, each sorted particle is
-// staged once as a record of its kernel weights and strength, and every mesh
-// node sums the records of the ns^2 stencil rows that cover it (each row one
-// contiguous range of records), in a fixed order.  No atomics touch the
-// mesh, so the result is deterministic run to run.
+// their stencil base index (bit-exact NINT) and counting-sorted by bin and,
+// inside a bin, by particle id, and every mesh node sums the particles of the
+// ns^2 stencil rows that cover it (each row one contiguous range), in a fixed
+// order: wavefronts that march over columns of nodes (k_p2m_march), or on a
+// small mesh a wavefront per line of nodes over records of each particle's
+// kernel weights and strength (k_p2m_stage, k_p2m_rows).  No atomics touch
+// the mesh, so the result is deterministic run to run.
 #pragma once
 #include <type_traits>
 

@@ -1,7 +1,7 @@
 // Compile-time specialised FFT engine (hot lengths).
 //
 // Same Stockham autosort algorithm as pm_fft.h, but the length, the radix
-// sequence, the threads per line P (a power of two) and the butterflies per
+// sequence, the threads per line P (a power of two, or L / 8) and the butterflies per
 // thread are template constants, so every index is folded, every register
 // array is statically indexed (no scratch) and a line that fits in one
 // wavefront (P <= 64) synchronises with wave-level fences instead of block

@@ -4,9 +4,7 @@
 //
 // Restates part_deriv_vorticity (vortex_codes/vortex_penalisation/source/
 // particle_derivatives/part_deriv_vorticity.f:57-115 for the 2nd-order and
-// :117-196 for the 4th-order stencils, :201-208 for the ghost map).  One
-// thread per component of an interior cell; the stencil neighbours along i
-// belong to nearby lanes, so the re-reads hit L1/L2.
+// :117-196 for the 4th-order stencils, :201-208 for the ghost map).
 // Every floating-point operation is an explicitly rounded one, in the order
 // the reference writes it, so the FP64 result is bit-identical to a
 // left-to-right evaluation of the reference's expressions.  Ghost cells of
