@@ -143,25 +143,46 @@ struct Kahan {
 // particle lies outside a periodic axis, where the reference zeroes every
 // weight) and its arrival rank in the bin (an atomic count: the order within a
 // bin is restored by particle id when the bin is staged)
-static __global__ void k_p2m_keys(PGeom g, const double *pos, NCount npc, int nbins, int *key, int *rank, int *count) {
+// Particles near the cell centres have neighbours in one bin, whose atomics on
+// one word wait for each other, so a run of neighbouring lanes of one bin adds
+// its length once.  What bounds it: the atomics' round trips.  56.6M particles,
+// 384^3: 727 us on average of a step's three calls and 1180 on the cell centres
+// with an atomic per particle, 444 and 458 so (32 B a particle, 1.8 GB); 2.1M
+// 34 -> 21 us.  (Four particles of a thread under way together: 549 us.)
+__device__ __forceinline__ int p2m_key(const PGeom &g, const double *x, int nbins) {
+  int b[3];
+  bool ok = true;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    b[d] = cell_index(x[d], g.xmin[d], g.c1dx[d]);
+    const int64_t bb = b[d];
+    if (bb - g.off + g.ns - 1 < g.lo[d] || bb - g.off > g.hi[d]) ok = false;
+    if (g.bc[d] != 0 && (x[d] < g.xmin[d] || x[d] > g.xmax[d])) ok = false;
+  }
+  return ok ? (b[0] - g.blo[0]) + g.nb[0] * ((b[1] - g.blo[1]) + g.nb[1] * (b[2] - g.blo[2])) : nbins;
+}
+static __global__ void k_p2m_keys(PGeom g, const double *__restrict__ pos, NCount npc, int nbins,
+                                  int *__restrict__ key, int *__restrict__ rank, int *__restrict__ count) {
   const int64_t np = npc.get();
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < np; q += (int64_t)gridDim.x * blockDim.x) {
-    int b[3];
-    bool ok = true;
-    for (int d = 0; d < 3; ++d) {
-      double x = pos[3 * q + d];
-      b[d] = cell_index(x, g.xmin[d], g.c1dx[d]);
-      const int64_t bb = b[d];
-      if (bb - g.off + g.ns - 1 < g.lo[d] || bb - g.off > g.hi[d]) ok = false;
-      if (g.bc[d] != 0 && (x < g.xmin[d] || x > g.xmax[d])) ok = false;
+  const int lane = threadIdx.x & 63;
+  // whole wavefronts: a lane past the end has no bin and stores nothing
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q - lane < np; q += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t p = q < np ? q : np - 1;
+    const double x[3] = {pos[3 * p], pos[3 * p + 1], pos[3 * p + 2]};
+    const int k = q < np ? p2m_key(g, x, nbins) : nbins;
+    // neighbouring lanes of one bin as one count, that of the first of them
+    const int before = __shfl_up(k, 1);
+    const uint64_t heads = __ballot(lane == 0 || before != k);
+    const uint64_t after = lane == 63 ? 0 : heads >> (lane + 1);
+    const int run = after ? __ffsll((unsigned long long)after) : 64 - lane;
+    int r = 0;
+    if (k < nbins && (heads >> lane & 1)) r = atomicAdd(&count[k], run);
+    const int head = lane - __clzll((long long)(heads << (63 - lane)));
+    r = __shfl(r, head) + lane - head;
+    if (q < np) {
+      key[q] = k;
+      rank[q] = r;
     }
-    int k = nbins, rk = 0;
-    if (ok) {
-      k = (b[0] - g.blo[0]) + g.nb[0] * ((b[1] - g.blo[1]) + g.nb[1] * (b[2] - g.blo[2]));
-      rk = atomicAdd(&count[k], 1);
-    }
-    key[q] = k;
-    rank[q] = rk;
   }
 }
 
