@@ -328,18 +328,37 @@ void particles_release() {
 // 96^3 161 / 148, 256^3 1926 / 910; M6* FP64 64^3 245 / 283, 72^3 455 / 277,
 // 112^3 1209 / 423; M6* FP32 64^3 163 / 282, 72^3 292 / 273, 160^3 2142 / 604.
 // (Above 64 nodes along x a node line is two wavefronts, which is where the
-// lines lose but for FP32 M'4, whose records are the smallest.)
+// lines lose but for FP32 M'4, whose records are the smallest.)  The rule knows
+// the mesh alone, so that a recorded step, whose count is on the device, adds
+// as an eager one does.  It costs FP32 M'4 sets that fill a few per cent of 90^3
+// to 120^3: cubes of 2 % on 96^3 77 / 90, on 112^3 94 / 115, on 128^3 106 / 106
+// (two rings 115 / 117, 145 / 131, 180 / 146).
 static bool p2m_marches(const PGeom &g, int prec) {
   const int64_t lines = (int64_t)((g.E[0] + 63) / 64) * g.E[1] * g.E[2];
-  return lines >= (prec == PMGPU_FP32 && g.ns == 4 ? 15000 : 8192);
+  return lines >= (prec == PMGPU_FP32 && g.ns == 4 ? 15600 : 8192);
 }
 
-// z nodes per marching wavefront.  More share a row's staging but take
-// registers: 167 for 3 (M'4), three wavefronts per SIMD; 231 for M6*, two.
-// 128^3 FP64 with 2, 3, 4: 216, 218, 220 us at each one's best chunk; M6*
-// 112 x 96 x 80 373 us with 2, 346 with 3.
-constexpr int kMarchQz = 3;
+// tiles that the grid is made for: those past a set's chunks end at once, but
+// their launch costs (256^3: 5,600 workgroups where 690 march)
+constexpr int64_t kMarchMostTiles = 24576;
 constexpr int kMarchMostY = 32;   // longest march: its NS - 1 extra rows cost 10%; 384^3 with 32 and 96: 2.98, 2.93 ms
+
+static MarchTiles march_tiles(const PGeom &g) {
+  MarchTiles mt{};
+  // equal segments of at most 64 nodes: with fewer than 62 a row's particles
+  // (one per bin after a remesh) take one pass of the lanes, not two
+  mt.nx = (g.E[0] + 63) / 64;
+  mt.width = (g.E[0] + mt.nx - 1) / mt.nx;
+  mt.nz = (g.E[2] + kMarchQz - 1) / kMarchQz;
+  mt.py = (g.nb[1] + kPartY - 1) / kPartY;
+  mt.pz = (g.nb[2] + kMarchQz - 1) / kMarchQz;
+  mt.resident = 1024 * (g.ns == 4 ? 3 : 2);
+  mt.ylow = 1;
+  mt.yhigh = kMarchMostY;
+  mt.yhigh = mt.chunk(g.E[1], (int64_t)mt.nx * mt.nz, mt.resident);
+  mt.ylow = (int)std::min<int64_t>(((int64_t)mt.nx * mt.nz * g.E[1] + kMarchMostTiles - 1) / kMarchMostTiles, mt.yhigh);
+  return mt;
+}
 
 // bytes of the staged records of np particles (0: the mesh's gather has none)
 static size_t p2m_record_bytes(const PGeom &g, int prec, int64_t np) {
@@ -351,23 +370,17 @@ template <typename T, int NS>
 static void p2m_gather(const PGeom &g, const double *xpart, const double *part, int64_t np, int *ids, PartWS &w,
                        int nbins, T *mesh, int accumulate, hipStream_t st) {
   const int *start = w.start.as<int>();
-  const int nx = (g.E[0] + 63) / 64;
-  if (np > 0) hipLaunchKernelGGL(k_p2m_binsort, grid_for(nbins), dim3(256), 0, st, start, nbins, ids);
-  if (np > 0 && p2m_marches(g, sizeof(T) == 8 ? PMGPU_FP64 : PMGPU_FP32)) {
-    // equal segments of at most 64 nodes: with fewer than 62 a row's particles
-    // (one per bin after a remesh) take one pass of the lanes, not two
-    const int width = (g.E[0] + nx - 1) / nx, nz = (g.E[2] + kMarchQz - 1) / kMarchQz;
-    // the shortest y chunks that the chip still holds at once (a second, nearly
-    // empty round of wavefronts costs most: 160^3 FP32 chunks of 8 nodes 313 us,
-    // of 9 266 us, of 12 290 us)
-    const int64_t lines = (int64_t)nx * nz, resident = 1024 * (NS == 4 ? 3 : 2);
-    const int64_t most = resident / lines > 1 ? resident / lines : 1;
-    const int yc = (int)std::min<int64_t>((g.E[1] + most - 1) / most, kMarchMostY);
-    const int ny = (g.E[1] + yc - 1) / yc;
-    const int64_t tiles = lines * ny;
-    hipLaunchKernelGGL((k_p2m_march<T, NS, kMarchQz>), dim3((unsigned)((tiles + kMarchWaves - 1) / kMarchWaves)),
-                       dim3(64 * kMarchWaves), 0, st, g, start, ids, xpart, part, width, nx, yc, ny, tiles, mesh,
-                       accumulate);
+  const bool march = np > 0 && p2m_marches(g, sizeof(T) == 8 ? PMGPU_FP64 : PMGPU_FP32);
+  MarchTiles mt{};
+  if (march) mt = march_tiles(g);
+  int *const filled = w.count.as<int>() + nbins + 1;
+  if (np > 0)
+    hipLaunchKernelGGL(k_p2m_binsort, grid_for(nbins), dim3(256), 0, st, g, start, nbins, ids, mt,
+                       march ? filled : nullptr);
+  if (march) {
+    const int64_t blocks = (mt.tiles(g.E[1], mt.ylow) + kMarchWaves - 1) / kMarchWaves;
+    hipLaunchKernelGGL((k_p2m_march<T, NS>), dim3((unsigned)(blocks + 8 * kMarchRuns)), dim3(64 * kMarchWaves), 0,
+                       st, g, start, ids, xpart, part, mt, (const int *)filled, mesh, accumulate);
     return;
   }
   // the records are planar with np + 1 records per field (the allocation
@@ -376,8 +389,8 @@ static void p2m_gather(const PGeom &g, const double *xpart, const double *part, 
   if (np > 0)
     hipLaunchKernelGGL((k_p2m_stage<T, NS>), grid_for(np), dim3(256), 0, st, g, xpart, part, ids, start, nbins,
                        w.rec.as<T>(), rs);
-  hipLaunchKernelGGL((k_p2m_rows<T, NS>), dim3(nx, g.E[1], g.E[2]), dim3(64), 0, st, g, start, w.rec.as<T>(), rs,
-                     mesh, accumulate);
+  hipLaunchKernelGGL((k_p2m_rows<T, NS>), dim3((g.E[0] + 63) / 64, g.E[1], g.E[2]), dim3(64), 0, st, g, start,
+                     w.rec.as<T>(), rs, mesh, accumulate);
 }
 
 int p2m_device(const pmgpu_geom *geom, int prec, const double *xpart, const double *part, int64_t np, void *mesh,
@@ -395,7 +408,7 @@ int p2m_device(const pmgpu_geom *geom, int prec, const double *xpart, const doub
   // counting sort by bin: count and rank (keys), scan, scatter; the stage
   // kernel restores id order inside each bin
   if (w.key.ensure(sizeof(int) * ((size_t)np + 1)) || w.ids.ensure(sizeof(int) * 2 * ((size_t)np + 1)) ||
-      w.count.ensure(sizeof(int) * (nbins + 1)) || w.start.ensure(sizeof(int) * (nbins + 1)))
+      w.count.ensure(sizeof(int) * (nbins + 2)) || w.start.ensure(sizeof(int) * (nbins + 1)))
     return -1;
   int *key = w.key.as<int>();
   int *rank = w.ids.as<int>(), *id_out = rank + np + 1;
@@ -1459,7 +1472,7 @@ struct VStep {
     PM_CHECK(cap < ((int64_t)1 << 31) && nbins < (1 << 30) && nn < ((int64_t)1 << 31),
              "pmgpu_vstep: capacity or mesh too large");
     if (w.key.ensure(sizeof(int) * ((size_t)cap + 1)) || w.ids.ensure(sizeof(int) * 2 * ((size_t)cap + 1)) ||
-        w.count.ensure(sizeof(int) * (nbins + 1)) || w.start.ensure(sizeof(int) * (nbins + 1)) ||
+        w.count.ensure(sizeof(int) * (nbins + 2)) || w.start.ensure(sizeof(int) * (nbins + 1)) ||
         w.rec.ensure(p2m_record_bytes(g, prec, cap)) || w.flag.ensure(sizeof(int) * (nn + 1)) ||
         w.offs.ensure(sizeof(int) * (nn + 1)))
       return -1;

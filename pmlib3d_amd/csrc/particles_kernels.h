@@ -161,9 +161,11 @@ __device__ __forceinline__ int p2m_key(const PGeom &g, const double *x, int nbin
   }
   return ok ? (b[0] - g.blo[0]) + g.nb[0] * ((b[1] - g.blo[1]) + g.nb[1] * (b[2] - g.blo[2])) : nbins;
 }
+// count[nbins + 1], the parts of the mesh that hold particles (k_p2m_binsort), is cleared.
 static __global__ void k_p2m_keys(PGeom g, const double *__restrict__ pos, NCount npc, int nbins,
                                   int *__restrict__ key, int *__restrict__ rank, int *__restrict__ count) {
   const int64_t np = npc.get();
+  if (blockIdx.x == 0 && threadIdx.x == 0) count[nbins + 1] = 0;
   const int lane = threadIdx.x & 63;
   // whole wavefronts: a lane past the end has no bin and stores nothing
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q - lane < np; q += (int64_t)gridDim.x * blockDim.x) {
@@ -244,13 +246,81 @@ template <typename T, int NS> struct PRec {
   static constexpr int kVal = 3 * NS, kBx = 3 * NS + 3;
 };
 
+// z nodes per marching wavefront (k_p2m_march).  More share a row's staging but
+// take registers: 167 for 3 (M'4), three wavefronts per SIMD; 231 for M6*, two.
+// 128^3 FP64 with 2, 3, 4: 216, 218, 220 us at each one's best chunk; M6*
+// 112 x 96 x 80 373 us with 2, 346 with 3.
+constexpr int kMarchQz = 3;
+constexpr int kPartY = 4, kPartBlocks = 256;
+constexpr int kMarchRuns = 8;   // march_block
+
+// The tiles of a march: nx segments of `width` x nodes, nz groups of kMarchQz z
+// nodes, and y chunks of ylow to yhigh nodes.  How much of the mesh holds
+// particles is counted in parts of one segment, kPartY bin rows along y and
+// kMarchQz along z (py, pz of them).  A set that fills 40 % of them or more takes
+// chunks of yhigh, the shortest with which all tiles are `resident` at most, the
+// wavefronts that the chip holds (a second, nearly empty round of wavefronts
+// costs most: 160^3 FP32 chunks of 8 nodes 313 us, of 9 266 us, of 12 290 us).
+// For one that fills less, and would leave most of those wavefronts without
+// particles, the chunks are so short that the tiles with particles are about
+// three quarters of `resident`.  A node's sums do not depend on its chunk.
+// Whole depositions, us, with chunks of yhigh for every set and now (a wavefront
+// per line of nodes: FP64, then FP32 M'4): a cube of 2 % of 256^3 FP64 680, 283
+// (980), FP32 655, 266 (525), of 10 % FP32 747, 432 (830); two rings on 128^3
+// FP32 188, 146 (180), 256^3 911, 530 (1250), 384^3 2445, 1550 (3617).
+struct MarchTiles {
+  int width, nx, nz, py, pz, resident, ylow, yhigh;
+  __host__ __device__ int parts() const { return nx * py * pz; }
+  __host__ __device__ bool fills(int filled) const { return 5 * filled >= 2 * parts(); }
+  __host__ __device__ int64_t tiles(int ey, int yc) const { return (int64_t)nx * nz * ((ey + yc - 1) / yc); }
+  // y chunk with which `used` columns of tiles are `most` tiles at most
+  __host__ __device__ int chunk(int ey, int64_t used, int most) const {
+    const int n = used > 0 && used < most ? (int)(most / used) : 1, yc = (ey + n - 1) / n;
+    return yc < ylow ? ylow : (yc > yhigh ? yhigh : yc);
+  }
+  // (below ns / 2 nodes a chunk's ns - 1 further rows cost more than the chip's
+  // idle SIMDs, unless there are as many of these as tiles)
+  __host__ __device__ int chunk_of(int ey, int ns, int filled) const {
+    if (fills(filled)) return yhigh;
+    const int64_t used = ((int64_t)nx * nz * filled + parts() - 1) / parts();
+    const int yc = chunk(ey, used, resident * 3 / 4), least = ns / 2 < yhigh ? ns / 2 : yhigh;
+    return yc < least && used * ey > 1024 * (int64_t)yc ? least : yc;
+  }
+  __device__ int runs(int filled) const { return min(parts() / max(filled, 1), kMarchRuns); }
+};
+
 // One thread per bin: order the bin's particles by id (the order a stable
 // sort by bin would give); bins of one particle, the usual case, do nothing.
-static __global__ void __launch_bounds__(256) k_p2m_binsort(const int *start, int nbins, int *ids) {
+// filled (or null): counts the parts of the mesh (MarchTiles) that hold a
+// particle, for the march that follows.
+static __global__ void __launch_bounds__(256) k_p2m_binsort(PGeom g, const int *start, int nbins, int *ids,
+                                                            MarchTiles mt, int *filled) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nbins; k += gridDim.x * blockDim.x) {
     const int t0 = start[k], n = start[k + 1] - t0;
     if (n > 1) sort_ids(ids + t0, n);
   }
+  // (as many blocks as the parts need, up to kPartBlocks: each adds to the one count once)
+  const int parts = mt.parts(), nblk = min((int)gridDim.x, min(kPartBlocks, (parts + 255) / 256));
+  if (!filled || (int)blockIdx.x >= nblk) return;
+  __shared__ int sum;
+  if (threadIdx.x == 0) sum = 0;
+  __syncthreads();
+  int n = 0;
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < parts; p += nblk * (int)blockDim.x) {
+    const int seg = p % mt.nx, r = p / mt.nx, by = r % mt.py * kPartY, bz = r / mt.py * kMarchQz;
+    const int x0 = seg * mt.width, xe = min(x0 + mt.width + g.ns - 1, g.nb[0]);
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < kPartY * kMarchQz; ++i) {
+      const int k = g.nb[0] * (min(by + i % kPartY, g.nb[1] - 1) + g.nb[1] * min(bz + i / kPartY, g.nb[2] - 1));
+      any |= start[k + xe] ^ start[k + x0];
+    }
+    n += any != 0;
+  }
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_down(n, o, 64);
+  if ((threadIdx.x & 63) == 0 && n) atomicAdd(&sum, n);
+  __syncthreads();
+  if (threadIdx.x == 0 && sum) atomicAdd(filled, sum);
 }
 
 // One thread per sorted particle t < start[nbins]: its record at slot t
@@ -526,12 +596,21 @@ struct RowData {
   double x[2][3], v[2][3];
 };
 
-template <typename T, int NS, int QZ>
+// Tile block of workgroup b, n in all: one run of consecutive blocks on each
+// XCD, whose rows they share in its L2, or, for particles in a part of the mesh,
+// up to kMarchRuns shorter ones, so that the part is work for every XCD.  Reaches
+// every block of [0, n) once for b < n + 8 kMarchRuns.
+__device__ __forceinline__ int64_t march_block(int64_t b, int64_t n, int runs) {
+  const int64_t len = (n + 8 * runs - 1) / (8 * runs), x = b % 8, k = b / 8;
+  return (k / len * 8 + x) * len + k % len;
+}
+
+template <typename T, int NS>
 __global__ void __launch_bounds__(64 * kMarchWaves)
     k_p2m_march(PGeom g, const int *__restrict__ start, const int *__restrict__ ids, const double *__restrict__ pos,
-                const double *__restrict__ val, int width, int nx, int ychunk, int ny, int64_t tiles,
-                T *__restrict__ mesh, int accumulate) {
-  constexpr int NR = QZ + NS - 1;   // bin rows per step
+                const double *__restrict__ val, MarchTiles mt, const int *__restrict__ filled, T *__restrict__ mesh,
+                int accumulate) {
+  constexpr int QZ = kMarchQz, NR = QZ + NS - 1;   // bin rows per step
   constexpr int NF = 3 * NS + 3;    // staged fields: x, y, z weights, strength
   __shared__ double lds_all[kMarchWaves][NF][kMarchCap];
   __shared__ int wxo_all[kMarchWaves][kMarchCap];
@@ -539,9 +618,13 @@ __global__ void __launch_bounds__(64 * kMarchWaves)
   double (*lds)[kMarchCap] = lds_all[wave];
   // lane 0's x weight (a slot the particle may not have), in words from its column
   int *wxo = wxo_all[wave];
-  // XCD-aware order: the wavefronts of one XCD take neighbouring columns (x
-  // fastest, then y, then z), whose rows they share in that XCD's L2
-  const int64_t lt = xcd_tile(blockIdx.x, gridDim.x) * kMarchWaves + __builtin_amdgcn_readfirstlane(wave);
+  // neighbouring columns, x fastest, then y, then z
+  const int width = mt.width, nx = mt.nx;
+  const int ychunk = mt.chunk_of(g.E[1], NS, *filled), ny = (g.E[1] + ychunk - 1) / ychunk;
+  const int64_t tiles = mt.tiles(g.E[1], ychunk);
+  const int64_t lt =
+      march_block(blockIdx.x, (tiles + kMarchWaves - 1) / kMarchWaves, mt.runs(*filled)) * kMarchWaves +
+      __builtin_amdgcn_readfirstlane(wave);
   if (lt >= tiles) return;
   const int x0 = (int)(lt % nx) * width;
   const int y0 = (int)((lt / nx) % ny) * ychunk, iz0 = (int)(lt / ((int64_t)nx * ny)) * QZ;
@@ -555,6 +638,24 @@ __global__ void __launch_bounds__(64 * kMarchWaves)
   auto row_key = [&](int by, int bzr) {
     return no_row(by, bzr) ? 0 : g.nb[0] * (by + g.nb[1] * (iz0 + bzr));
   };
+  // no particle reaches the tile: its nodes take zeros, without a march (not
+  // looked for in a set that fills the mesh)
+  bool some = mt.fills(*filled);
+  if (!some)
+    for (int i = lane; i < (y1 - y0 + NS - 1) * NR; i += 64) {
+      const int k = row_key(y0 + i / NR, i % NR);
+      some = some || (!no_row(y0 + i / NR, i % NR) && start[k + xe] != start[k + x0]);
+    }
+  if (!__any(some)) {
+    const int words = 3 * min(width, g.E[0] - x0);
+    for (int r = 0; r < (y1 - y0) * QZ; ++r) {
+      const int iy = y0 + r / QZ, iz = iz0 + r % QZ;
+      if (iz >= g.E[2]) continue;
+      T *m = mesh + 3 * ((int64_t)x0 + (int64_t)g.E[0] * (iy + (int64_t)g.E[1] * iz));
+      for (int c = lane; c < words; c += 64) m[c] = accumulate ? (T)((double)m[c] + 0.0) : (T)0;
+    }
+    return;
+  }
   double acc[NS][QZ][3];
 #pragma unroll
   for (int j = 0; j < NS; ++j)
