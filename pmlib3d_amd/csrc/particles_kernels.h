@@ -330,8 +330,8 @@ template <typename T, int NS>
 __global__ void __launch_bounds__(256) k_p2m_stage(PGeom g, const double *pos, const double *val, const int *ids,
                                                    const int *start, int nbins, T *rec, int64_t rs) {
   const int nvalid = start[nbins];
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nvalid; t += gridDim.x * blockDim.x) {
-    const int q = ids[t];
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < nvalid; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t q = ids[t];   // (3 q passes 2^31 from 715,827,883 particles on)
     T wt[3 * NS];
     int bx = 0;
 #pragma unroll
