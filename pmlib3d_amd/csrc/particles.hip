@@ -717,12 +717,11 @@ struct MapBox {
   int per[3];
 };
 // code[q]: the classes of particle q.  tsum, counts[1..3]: the totals of axis 0
-// per tile and in all; counts[4]: set if a particle is still outside after one
-// wrap; counts[8]: a bit for each axis that someone leaves
+// per tile and in all; counts[8]: a bit for each axis that someone leaves
 __global__ void __launch_bounds__(kPartThreads) k_map_classify(int64_t n, const double *pos, MapBox box, uint8_t *code,
                                                                Mig3 *tsum, int *counts) {
   Mig3 s{0, 0, 0};
-  int axes = 0, again = 0;
+  int axes = 0;
 #pragma unroll
   for (int j = 0; j < kPartItems; ++j) {
     const int64_t q = (int64_t)blockIdx.x * kPartTile + j * kPartThreads + threadIdx.x;
@@ -734,12 +733,7 @@ __global__ void __launch_bounds__(kPartThreads) k_map_classify(int64_t n, const 
       int c = x < box.lo[d] ? 1 : (x >= box.hi[d] ? 2 : 0);
       if (c != 0) {
         axes |= 1 << d;
-        if (box.per[d]) {
-          const double y = c == 1 ? x + box.len[d] : x - box.len[d];
-          if (y < box.lo[d] || y >= box.hi[d]) again = 1;
-        } else {
-          c = 3;
-        }
+        if (!box.per[d]) c = 3;
       }
       cc |= c << (2 * d);
     }
@@ -748,7 +742,6 @@ __global__ void __launch_bounds__(kPartThreads) k_map_classify(int64_t n, const 
   }
   Mig3 tot;
   (void)block_scan3(s, tot);
-  if (again) atomicOr(&counts[4], 1);
   int any = 0;
 #pragma unroll
   for (int d = 0; d < 3; ++d)
@@ -917,10 +910,10 @@ static int drop_particles(PartWS &w, int64_t n, int64_t out, const PBox &box, do
   return rows_back(n - out, dst, src, narr, st);
 }
 
-// the map by classes (k_map_classify) of n particles of which some are outside;
-// *general: a particle needs more than one wrap, nothing was done
+// the map by classes (k_map_classify) of n particles of which some are outside,
+// none of them after one wrap
 static int map_particles(PartWS &w, const pmgpu_geom *geom, int64_t n, double **arr, double **spare, int narr,
-                         int64_t *np_out, int *in_spare, bool *general, hipStream_t st) {
+                         int64_t *np_out, int *in_spare, hipStream_t st) {
   MapBox box;
   for (int d = 0; d < 3; ++d) {
     box.lo[d] = geom->xmin[d];
@@ -934,15 +927,13 @@ static int map_particles(PartWS &w, const pmgpu_geom *geom, int64_t n, double **
   int *list[2] = {w.cls.as<int>(), w.cls.as<int>() + ni};
   uint8_t *code[2] = {reinterpret_cast<uint8_t *>(list[1] + ni), reinterpret_cast<uint8_t *>(list[1] + ni) + ni};
   Mig3 *tsum = reinterpret_cast<Mig3 *>(code[1] + ni);
-  int *counts = w.count.as<int>();   // four per axis; counts[4] and [8] as in k_map_classify
+  int *counts = w.count.as<int>();   // four per axis; counts[8] as in k_map_classify
   PM_HIP(hipMemsetAsync(counts, 0, sizeof(int) * 12, st));
   hipLaunchKernelGGL(k_map_classify, dim3(tiles(n)), dim3(kPartThreads), 0, st, n, (const double *)arr[0], box, code[0],
                      tsum, counts);
   int got[12];
   PM_HIP(hipMemcpyAsync(got, counts, sizeof(got), hipMemcpyDeviceToHost, st));
   PM_HIP(hipStreamSynchronize(st));
-  *general = got[4] != 0;
-  if (*general) return 0;
   *np_out = n;
   int cur = 0;
   bool listed = false;
@@ -1015,6 +1006,7 @@ int advance_device(const pmgpu_geom *geom, int rk_order, int stage, double dt, i
     for (int d = 0; d < 3; ++d) {
       box.lo[d] = geom->xmin[d];
       box.hi[d] = geom->xmax[d];
+      box.len[d] = geom->bound_cond[d] != 0 ? geom->xmax[d] - geom->xmin[d] : 0.0;
     }
     const bool all_free = geom->bound_cond[0] == 0 && geom->bound_cond[1] == 0 && geom->bound_cond[2] == 0;
     const int nt = (int)((n + kPartTile - 1) / kPartTile);
@@ -1035,10 +1027,10 @@ int advance_device(const pmgpu_geom *geom, int rk_order, int stage, double dt, i
     }
     if (all_free)
       return drop_particles(w, n, any[3], box, arr, spare, rk_order > 1 ? (rhs ? 4 : 3) : 2, np_out, in_spare, st);
-    bool general;
-    if (map_particles(w, geom, n, arr, spare, rk_order > 1 ? (rhs ? 4 : 3) : 2, np_out, in_spare, &general, st))
-      return -1;
-    if (!general) return 0;
+    // (particles several periods away go on to the partitions of an axis that
+    // wrap as often as it takes; the update knows, so that they classify once)
+    if (!(any[0] & 2))
+      return map_particles(w, geom, n, arr, spare, rk_order > 1 ? (rhs ? 4 : 3) : 2, np_out, in_spare, st);
   }
   const int narr = rk_order > 1 ? (rhs ? 4 : 3) : 2;
   const int64_t n0 = n;
@@ -1562,7 +1554,7 @@ struct VStep {
                              (const double *)A.a[0], n, A.a[1]);
       }
       const RkCoef k = rk_coef(rk, s, 0);
-      PBox box;
+      PBox box{};
       for (int d = 0; d < 3; ++d) {
         box.lo[d] = geom.xmin[d];
         box.hi[d] = geom.xmax[d];

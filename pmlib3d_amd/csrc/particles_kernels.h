@@ -1176,13 +1176,15 @@ struct RkCoef {
   double a1, b1, c1, a2, b2, c2;
 };
 
-// the patch box [lo, hi) per axis
+// the patch box [lo, hi) per axis; len: the period of a periodic axis, 0 on a
+// free one (or where only outside or not is asked)
 struct PBox {
-  double lo[3], hi[3];
+  double lo[3], hi[3], len[3];
 };
 
 // the RK stage update of every particle word; with `outside` given, also
-// flags (1) a particle that the update leaves outside the box on any axis
+// flags a particle that the update leaves outside the box on any axis (bit 1),
+// and one that is still outside after one wrap of a periodic axis (bit 2)
 // dvort null: a zero right-hand side (dvort = dvort_rk = +0), dvort_rk is
 // neither read nor written and vort takes the increment c2 dr that the full
 // form rounds for those zeros, dr = a2 (+0) + (b2 dt) (+0)
@@ -1212,7 +1214,11 @@ static __global__ void k_rk_update(RkCoef k, double dt, NCount npc, double *pos,
     if (outside) {
       const bool o = x < box.lo[d] || x >= box.hi[d];
       const uint64_t m = __ballot(o);
-      if (m && (threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1) atomicOr(outside, 1);
+      if (m) {
+        const double y = x < box.lo[d] ? x + box.len[d] : x - box.len[d];
+        const bool far = __any(o && box.len[d] != 0.0 && (y < box.lo[d] || y >= box.hi[d]));
+        if ((threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1) atomicOr(outside, far ? 3 : 1);
+      }
     }
   }
 }
