@@ -55,7 +55,6 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 constexpr int kTx = 64, kTy = 8;
-constexpr int kZc = 32;   // most planes per workgroup
 
 // A workgroup of kTx x kTy threads owns an (i, j) tile of interior cells and
 // walks the planes of its z chunk (zc planes).  Per plane it forms f once for
@@ -253,13 +252,27 @@ __global__ void __launch_bounds__(256) k_penalise_sums(const double *partial, in
 
 constexpr int kMaxDevices = 64;
 
-// workgroups of k_penalise: chunks of kZc planes, fewer on a mesh that leaves
-// CUs idle (two workgroups per CU; each chunk re-reads fd planes)
-static dim3 penalise_grid(const pmgpu_geom *geom, int &zc) {
-  const int64_t tiles = (int64_t)((geom->ncell[0] + kTx - 1) / kTx) * ((geom->ncell[1] + kTy - 1) / kTy);
-  zc = kZc;
-  while (zc > 4 && tiles * ((geom->ncell[2] + zc - 1) / zc) < 512) zc /= 2;
-  return dim3((geom->ncell[0] + kTx - 1) / kTx, (geom->ncell[1] + kTy - 1) / kTy, (geom->ncell[2] + zc - 1) / zc);
+// Workgroups of k_penalise.  A chunk of zc planes costs the loads of zc + fd,
+// and the chip takes `slots` workgroups at a time (two on a CU in FP64, three in
+// FP32), so zc is the one of 64, 32 .. 4 with the least rounds x (zc + fd), of
+// equal ones the smallest (but not 4: more sums to add).  With the largest zc <=
+// 32 that gives 512 workgroups instead, and now, us without the sums: FP64 4th
+// order 160^3 88, 79; 200^3 243, 203; 256^3 312, 288; FP32 224^3 181, 154; 256^3
+// 222, 192; FP32 2nd order 256^3 209, 177 (64 x 4 tiles of 16 planes, which lose
+// with the sums, 330 to 212: 161).
+static dim3 penalise_grid(const pmgpu_geom *geom, int fd, bool f32, int &zc) {
+  const int nx = (geom->ncell[0] + kTx - 1) / kTx, ny = (geom->ncell[1] + kTy - 1) / kTy;
+  const int64_t slots = 256 * (f32 ? 3 : 2);
+  int64_t best = 0;
+  for (int c = 64; c >= 4; c /= 2) {
+    const int64_t blocks = (int64_t)nx * ny * ((geom->ncell[2] + c - 1) / c);
+    const int64_t cost = (blocks + slots - 1) / slots * (c + fd);
+    if (best == 0 || cost < best || (cost == best && c >= 8)) {
+      best = cost;
+      zc = c;
+    }
+  }
+  return dim3(nx, ny, (geom->ncell[2] + zc - 1) / zc);
 }
 // partial sums a call may need (one per workgroup) and the limit of the calls
 // with a fixed buffer: one per 64 x 4 cells of a plane
@@ -317,7 +330,7 @@ static int penalise_run(const pmgpu_geom *geom, const void *vel, const void *chi
   a.cz = T(1.0) / (T(2.0) * T(geom->dx[2]));
   a.vort = (T *)vort;
   PM_CHECK(geom->ncell[2] < 65536 && geom->ncell[1] < (1 << 20), "pmgpu_penalise: mesh too large");
-  const dim3 grid = penalise_grid(geom, a.zc);
+  const dim3 grid = penalise_grid(geom, fd_order, sizeof(T) == 4, a.zc);
   const int64_t nb = (int64_t)grid.x * grid.y * grid.z;
   PM_CHECK(!partial || partial_blocks(geom) <= cap, "pmgpu_penalise: more blocks than the partial-sum buffer holds");
   a.partial = partial;
