@@ -525,16 +525,17 @@ __device__ __forceinline__ double2 buf_load(__amdgpu_buffer_rsrc_t r, int voff, 
 // FIELD: the velocity in place (kVel; kVelFiltered: with every axis periodic
 // the spectral G carries the filter zeta as well when the vorticity is
 // filtered, poisson/pmlib_poisson_solve.f:339-349), or psi-hat = G w-hat or
-// zeta w-hat [+ reprojection] into their own spectra (:767-872).  A solve with
-// more outputs than the velocity launches the others first: a forward
-// transform more for each, but a kernel that forms them all keeps its spectra
-// in registers or LDS at one wavefront per SIMD (256^3 FP64 velocity and
-// vorticity 3.25 ms, in two launches 2.30; 64^3 FP64 velocity and psi 58, 47 us).
-// (The vorticity in FP64 is held to two wavefronts per SIMD at 4 to 20 spilled
-// registers: 2.06 -> 1.43 ms.)
-constexpr int kVel = 0, kPsi = 1, kVort = 2, kVelFiltered = 3;
+// zeta w-hat [+ reprojection] into their own spectra (:767-872), or kEach, the
+// requested ones in turn, tile by tile, the velocity last (a thread reads the
+// words of the spectrum that it writes).  A field has a forward transform of its
+// own: a kernel that forms them all from one keeps its spectra in registers or
+// LDS at one wavefront per SIMD (256^3 FP64 velocity and vorticity 3.25 ms, in
+// two passes 2.30; 64^3 FP64 velocity and psi 58, 47 us).  (The vorticity in FP64
+// is held to two wavefronts per SIMD at 4 to 20 spilled registers: 2.06 -> 1.43
+// ms.)
+constexpr int kVel = 0, kPsi = 1, kVort = 2, kVelFiltered = 3, kEach = 4;
 template <typename R, int L, int TC, bool ALLPER, bool HALF, int FIELD>
-__global__ void __launch_bounds__(RGeo<L>::P *TC, sizeof(R) == 8 && FIELD == kVort ? 2 : 1)
+__global__ void __launch_bounds__(RGeo<L>::P *TC, sizeof(R) == 8 && (FIELD == kVort || FIELD == kEach) ? 2 : 1)
     k_z3_r(ZArgs a, const cplx_t<R> *tw_all) {
   using V = cplx_t<R>;
   constexpr int K = reg_key(L), P = Geo<K>::P, E = L / P;
@@ -557,103 +558,28 @@ __global__ void __launch_bounds__(RGeo<L>::P *TC, sizeof(R) == 8 && FIELD == kVo
   const uint32_t extent = (uint32_t)((a.Mz - 1) * rsb + (int64_t)ncols_here * 3 * sizeof(V));
   const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(base, extent);
   const int voff = (int)(p * rsb) + col * 3 * (int)sizeof(V);
-  V w[3][E];
-#pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const bool ok = col_ok && (HALF ? m < E / 2 : p + P * m < a.Mz);
-    const int soff = (int)((int64_t)P * m * rsb);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-      w[c][m] = ok ? buf_load(rsrc, voff + c * (int)sizeof(V), soff, V{}) : cmake<V>(0, 0);
-  }
-  V *line = lds + col * ST;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) fft_regs<K, -1, V, HALF, false, 1>(w[c], line, p, twd);
-  // u-hat = G 2 pi i (k x w-hat); Nyquist wavenumbers drop out (Hermitian
-  // projection of the real inverse); the 1 / L of the inverse transform
-  // rides on the same factor
-  const R ki = wavenumber<R>(kx, a.Lx, a.dk[0], a.ksmp[0]);
-  const R kj = wavenumber<R>(ky, a.Ly, a.dk[1], a.ksmp[1]);
-  const bool nx = 2 * kx == a.Lx, ny = 2 * ky == a.Ly;
-  const R kx_ = nx ? (R)0 : ki, ky_ = ny ? (R)0 : kj;
-  const int kyf = ky <= a.Ly - ky ? ky : a.Ly - ky;
-  const R pi = (R)3.14159265358979323846, inv_l = (R)1 / (R)L;
-  const R twopi = (R)6.28318530717958647692 / (R)L;
-  // G-hat of the thread's rows, all loads issued before any is used (a
-  // column past Hx reads column 0 and is masked)
-  const R *G = reinterpret_cast<const R *>(a.Ghat) + (int64_t)kyf * a.Hx + (col_ok ? kx : 0);
-  const int64_t gz = (int64_t)a.Hy * a.Hx;
-  R gv[E];
-  if constexpr (!ALLPER) {
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-      const int n = p + P * m;
-      const int kzf = n <= L - n ? n : L - n;
-      gv[m] = G[kzf * gz];
+  if constexpr (FIELD != kEach) {
+    constexpr int F = FIELD;
+#include "poisson_z3_field.h"
+  } else {
+    if (a.want_psi) {
+      constexpr int F = kPsi;
+#include "poisson_z3_field.h"
+      __syncthreads();
     }
-  }
-#pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int n = p + P * m;
-    const R kk = wavenumber<R>(n, L, a.dk[2], a.ksmp[2]);
-    R zeta = (R)1, g;
-    if (FIELD == kVort || FIELD == kVelFiltered || (FIELD == kPsi && ALLPER && a.want_vort))
-      zeta = zeta_filter<R>(a.order, (R)a.eps2pi * sqrt(ki * ki + kj * kj + kk * kk));
-    if constexpr (ALLPER) {
-      const R kmag = ki * ki + kj * kj + kk * kk;
-      g = kmag > (R)0 ? zeta / ((R)4 * (pi * pi) * kmag) : (R)0;
-    } else {
-      g = col_ok ? gv[m] * (R)a.h3 : (R)0;
-    }
-    const bool nz = 2 * n == L;
-    const V w0 = w[0][m], w1 = w[1][m], w2 = w[2][m];
-    if constexpr (FIELD == kVel || FIELD == kVelFiltered) {
-      const R kz_ = nz ? (R)0 : kk;
-      const V c0 = csub(cscale(w2, ky_), cscale(w1, kz_));
-      const V c1 = csub(cscale(w0, kz_), cscale(w2, kx_));
-      const V c2 = csub(cscale(w1, kx_), cscale(w0, ky_));
-      const R f = g * twopi;
-      w[0][m] = cmake<V>(-c0.y * f, c0.x * f);
-      w[1][m] = cmake<V>(-c1.y * f, c1.x * f);
-      w[2][m] = cmake<V>(-c2.y * f, c2.x * f);
-    } else if constexpr (FIELD == kPsi) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) w[c][m] = cscale(w[c][m], g * inv_l);
-    } else {
-      // reprojection: -4 pi^2 G k_c sum_d k_d w_d over the pairs (c, d) of
-      // equal Nyquist parity (:861-872)
-      const R kd[3] = {ki, kj, kk};
-      const bool nd[3] = {nx, ny, nz};
-      const R f = a.reproj ? -(R)4 * (pi * pi) * g * inv_l : (R)0;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const V wc = c == 0 ? w0 : (c == 1 ? w1 : w2);
-        V q = cscale(wc, zeta * inv_l);
-        if (a.reproj) {
-          V acc = cmake<V>(0, 0);
-          if (nd[0] == nd[c]) acc = cadd(acc, cscale(w0, ki));
-          if (nd[1] == nd[c]) acc = cadd(acc, cscale(w1, kj));
-          if (nd[2] == nd[c]) acc = cadd(acc, cscale(w2, kk));
-          q = cadd(q, cscale(acc, f * kd[c]));
-        }
-        w[c][m] = q;
+    if (a.want_vort) {
+      {
+        constexpr int F = kVort;
+#include "poisson_z3_field.h"
       }
+      __syncthreads();
     }
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) fft_regs<K, 1, V, false, HALF, 1>(w[c], line, p, twd);
-  // Stores are plain global stores: buffer-resource stores of these
-  // 8-byte-aligned records, which the compiler merges into 16-byte stores
-  // across components, have returned corrupted first components.
-  if (col_ok) {
-    V *out = FIELD == kPsi ? reinterpret_cast<V *>(a.Bpsi) : reinterpret_cast<V *>(FIELD == kVort ? a.Bvort : a.B);
-    V *dst = out + (int64_t)ky * a.kys + (int64_t)kx0 * 3 + (int64_t)p * a.rs + col * 3;
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-      if (HALF ? m < E / 2 : p + P * m < a.Mz) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) dst[(int64_t)P * m * a.rs + c] = w[c][m];
-      }
+    if (ALLPER && a.want_vort) {
+      constexpr int F = ALLPER ? kVelFiltered : kVel;
+#include "poisson_z3_field.h"
+    } else {
+      constexpr int F = kVel;
+#include "poisson_z3_field.h"
     }
   }
 }

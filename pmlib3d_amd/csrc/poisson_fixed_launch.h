@@ -107,18 +107,36 @@ template <typename R, int L> int zr_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipS
     default: return 0;
   }
 }
-// the velocity (last: in place) with the stream function and/or the vorticity
+// the velocity with the stream function and/or the vorticity: in one launch, or
+// in a launch for each, the velocity (in place) last.  One launch reads a tile
+// again while it is still in a cache and leaves no gaps, but its registers are
+// those of the neediest field.  us, a launch each and one launch: 32^3 FP32 all
+// outputs free 60, 55; 128^3 periodic FP32 psi 127, 120; 192^3 free FP64 all 3499,
+// 3195; but 160^3 free FP32 psi 625, 755, 256^3 free FP32 psi 2260, 2320, and, with
+// the vorticity's spills, 192^3 periodic FP64 691, 759.  Lines of 640 and more
+// take two columns a block (128 x 128 x 384 free FP64 all 3271, with four 3036,
+// with two 2825).
+constexpr int kFewBlocks = 1200;   // a launch that the chip takes at once
 template <typename R, int L> int zrx_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
-  if (a.want_psi) {
-    const int r = zr_T<R, L, 4, kPsi>(a, Ly, tw, st);
-    if (r != 1) return r;
+  constexpr bool pow2 = reg_key(L) == L;
+  constexpr int TC = L >= 640 ? 2 : 4;
+  if constexpr (!pow2 || L == 512) {
+    const bool few = (int64_t)((a.Hx + 3) / 4) * Ly <= kFewBlocks;
+    const bool spills = !pow2 && sizeof(R) == 8 && a.allper && a.want_vort;
+    if (spills || !(few || L >= 640 || (pow2 ? a.allper : sizeof(R) == 8 && !a.allper))) {
+      if (a.want_psi) {
+        const int r = zr_T<R, L, 4, kPsi>(a, Ly, tw, st);
+        if (r != 1) return r;
+      }
+      if (a.want_vort) {
+        const int r = zr_T<R, L, 4, kVort>(a, Ly, tw, st);
+        if (r != 1) return r;
+        if (a.allper) return zr_T<R, L, 4, kVelFiltered>(a, Ly, tw, st);
+      }
+      return zr_T<R, L, 4, kVel>(a, Ly, tw, st);
+    }
   }
-  if (a.want_vort) {
-    const int r = zr_T<R, L, 4, kVort>(a, Ly, tw, st);
-    if (r != 1) return r;
-    if (a.allper) return zr_T<R, L, 4, kVelFiltered>(a, Ly, tw, st);
-  }
-  return zr_T<R, L, 4, kVel>(a, Ly, tw, st);
+  return zr_T<R, L, TC, kEach>(a, Ly, tw, st);
 }
 
 template <typename R, int L> int z_L(ZArgs a, int Ly, const cplx_t<R> *tw, hipStream_t st) {
