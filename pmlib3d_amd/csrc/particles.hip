@@ -375,8 +375,8 @@ static void p2m_gather(const PGeom &g, const double *xpart, const double *part, 
   if (march) mt = march_tiles(g);
   int *const filled = w.count.as<int>() + nbins + 1;
   if (np > 0)
-    hipLaunchKernelGGL(k_p2m_binsort, grid_for(nbins), dim3(256), 0, st, g, start, nbins, ids, mt,
-                       march ? filled : nullptr);
+    hipLaunchKernelGGL(k_p2m_binsort, dim3(grid_for(nbins).x + (march ? mt.part_blocks() : 0)), dim3(256), 0, st, g,
+                       start, nbins, ids, mt, march ? filled : nullptr);
   if (march) {
     const int64_t blocks = (mt.tiles(g.E[1], mt.ylow) + kMarchWaves - 1) / kMarchWaves;
     hipLaunchKernelGGL((k_p2m_march<T, NS>), dim3((unsigned)(blocks + 8 * kMarchRuns)), dim3(64 * kMarchWaves), 0,
