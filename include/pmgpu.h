@@ -136,11 +136,20 @@ int pmgpu_poisson_batch_destroy(pmgpu_poisson_batch_t b);
  * Particles.  Particle arrays are (3, np) FP64 everywhere (positions in FP64
  * keep the particle -> cell index exact).  The host entry points use FP64
  * meshes; the *_device variants take device pointers, a hipStream_t (NULL:
- * the default stream) and the mesh precision: PMGPU_FP64 reproduces the
- * reference's arithmetic, PMGPU_FP32 uses an FP32 mesh with FP32 kernel
- * weights, compensated FP32 sums in deposition (each stencil row's terms of
- * a node fused into one FP32 partial, the row partials Kahan-added) and FP64
- * sums of the weighted FP32 node values in the gather.
+ * the default stream) and the mesh precision.
+ * Gather, advance, map and remesh: PMGPU_FP64 reproduces the reference's
+ * arithmetic bit for bit; PMGPU_FP32 gathers with FP32 kernel weights and FP64
+ * sums of the weighted FP32 node values.
+ * Deposition adds a node's particles stencil row by stencil row, not in the
+ * reference's order of particles, and equals it to rounding (1e-12 of the
+ * largest value in FP64).  The form depends on the mesh alone.  On meshes of at
+ * least 8192 lines of 64 nodes along x, ceil(E0 / 64) E1 E2 (15600 for
+ * PMGPU_FP32 with M'4): FP64 weights (M'4: fused multiply-adds) and fused FP64
+ * sums in both precisions, rounded once to the mesh (FP32: about 2.5e-8 from
+ * FP64).  On smaller meshes: PMGPU_FP64 weights and products rounded as the
+ * reference's; PMGPU_FP32 weights in FP32, each row's terms of a node fused
+ * into one FP32 partial and the row partials Kahan-added (about 1.5e-7 from
+ * FP64 with M'4, 2.8e-7 with M6*).
  * ------------------------------------------------------------------------ */
 
 /* Replaces pmlib_interp_particle_mesh(topo, xpart, part, mesh, ierr, clear,

@@ -1321,7 +1321,7 @@ struct Arr6 {
 // tile's own block scans in index order, from the sums before it (added by the
 // tile itself up to kPartFew tiles, beyond that by k_part_tile_scan).  A step
 // is bound by its launches, some 3 us each: three per axis (count, move, copy
-// back with the check) and one per stage for eight per axis and one per stage
+// back with the check) and one per stage, where there were seven per axis
 // (64^3 FP32, four steps: 1.93 -> 1.53 ms).
 // counters of a stage, zero at its start
 struct StageState {

@@ -583,7 +583,11 @@ __global__ void __launch_bounds__(64) k_p2m_rows(PGeom g, const int *start, cons
 // ascending in by, then bz; particles by bin, then id): deterministic, no
 // atomics on the mesh.
 // What bounds it: vector issue, about 3 + 3 nz + 3 ns nz operations per
-// particle and row, times the fullest lane's particle count over the mean.
+// particle and row, is half of it (128^3 M'4: 60 M wavefront instructions on
+// 1,024 SIMDs, 97 us on average and 108 on a SIMD with three wavefronts, of
+// 187); the rest is latency, since one round of two or three wavefronts per
+// SIMD leaves nothing to fill a stalled or finished one, and lanes that wait
+// for the fullest of their row.
 constexpr int kMarchWaves = 4;   // per block, one for each SIMD of a CU (they share nothing; 128^3 one: 243 us, four: 218)
 constexpr int kMarchCap = 96;   // particles of a row staged at a time (lanes below 32 take two)
 
@@ -877,9 +881,12 @@ template <typename T> __global__ void k_halo_add(T *m, PGeom g, int d) {
 // What bounds it: the L1, which takes about 16 cycles per load instruction of a
 // wavefront, however narrow.  A stencil row's ns nodes lie side by side, so a
 // row is read as the one run of 3 ns words they make (M'4: 6 dwordx4 in FP64, 3
-// in FP32) instead of node by node (8 and 4 loads).  us before and now: 128^3 FP64
-// M'4 periodic 191, 149, free 189, 155; M6* free 572, 475; FP32 M'4 92, 75 and
-// 104, 97; M6* free 322, 283; 384^3 FP32 2270, 2020.
+// in FP32) instead of node by node (8 and 4 loads).  us before and now, a full
+// set moved by a smooth flow of up to half a cell: 128^3 FP64 M'4 periodic 191,
+// 149, free 189, 155; M6* free 572, 475; FP32 M'4 92, 75 and 104, 97; M6* free
+// 322, 283; 384^3 FP32 2270, 2020.  The gathers of a two-ring step from
+// jittered centres: 128^3 free FP64 244, 189, FP32 126, 118.
+// (64^3 FP32 M6* free: 52, 56; its clamped lanes are a larger share.)
 // Wavefronts with a stencil that leaves the mesh along x (clamped indices) move
 // those lanes' runs inside and their x weights along.
 // a stencil row: 3 ns words side by side, read 16 bytes at a time from any word
